@@ -822,26 +822,30 @@ static int fw_pass(RqCtx *c, Pass *P, float *out) {
             ptr[(size_t)l * n + b] = seq_layer(P->seq[b], l, 0);
             ptr[(size_t)(L + l) * n + b] = seq_layer(P->seq[b], l, 1);
         }
-    /* the items in six groups, each launched with its own query-vector bound: the f16 caches', then the bf16
-     * caches'; in each, the row blocks of <= 4 query vectors (decode rows: the narrow kernel, two blocks per CU), then
-     * the wider ones (prompt row blocks). A pass of both kinds of rows would otherwise run every decode row's items in
-     * the 16-vector kernel. Then the f32 and quantized caches', and the dot-product types' (k_attn_q) */
+    /* the items in six groups, a launch each: the f16 caches', the bf16 caches', each split into single rows of at most 4
+     * query vectors (decode rows: their own kernel) and the others; the f32 and quantized caches', the dot-product
+     * types' (k_attn_q). The row blocks of one sequence next to each other (the kv heads inside them, one
+     * per XCD where there are 8) for each key block in turn, so a key block's K / V are read again while they are in L2 */
     Item *it = (Item *)(h + o_items);
-    int gcnt[6] = { 0, 0, 0, 0, 0, 0 }, gnq[6] = { 1, 1, 1, 1, 1, 1 };
+    int gcnt[6] = { 0, 0, 0, 0, 0, 0 };
+#define RB_END(e, b) while (e < n && e - b < ROWS_OF(kvt[b]) && P->seq[e] == P->seq[b] && P->pos[e] == P->pos[e - 1] + 1) e++
     for (int grp = 0, k = 0; grp < 6; grp++)
         for (int b = 0; b < n;) {
-            int e = b + 1;
-            while (e < n && e - b < ROWS_OF(kvt[b]) && P->seq[e] == P->seq[b] && P->pos[e] == P->pos[e - 1] + 1) e++;
-            int nb = (P->pos[e - 1] + 1 + GW_ATT_P - 1) / GW_ATT_P, nq = (e - b) * kv_mul;
-            int kg = gw_kv_dot(kvt[b]) ? 5 : gw_kv_att_q(kvt[b]) ? 4 : 2 * (kvt[b] == RQ_KV_BF16) + (nq > 4);
-            if (kg == grp) {
-                for (int g = 0; g < nkv; g++)
-                    for (int kb = 0; kb < nb; kb++) it[k++] = (Item){ b, e - b, g, kb };
-                gcnt[grp] += nkv * nb;
-                gnq[grp] = nq > gnq[grp] ? nq : gnq[grp];
-            }
-            b = e;
+            int se = b + 1; /* (the sequence's rows: b .. se - 1) */
+            while (se < n && P->seq[se] == P->seq[b]) se++;
+            const int kg = gw_kv_dot(kvt[b]) ? 5 : gw_kv_att_q(kvt[b]) ? 4 : 2 * (kvt[b] == RQ_KV_BF16) + (se - b > 1 || kv_mul > 4);
+            const int nbs = P->pos[se - 1] / GW_ATT_P + 1;
+            for (int kb = 0; kb < nbs && kg == grp; kb++)
+                for (int r = b; r < se;) {
+                    int e = r + 1;
+                    RB_END(e, r);
+                    if (kb * GW_ATT_P <= P->pos[e - 1])
+                        for (int g = 0; g < nkv; g++) it[k++] = (Item){ r, e - r, g, kb }, gcnt[grp]++;
+                    r = e;
+                }
+            b = se;
         }
+#undef RB_END
 #undef ROWS_OF
     HIPCHK(c, "hipMemcpyAsync (pass metadata)", hipMemcpyAsync(d, h, total, hipMemcpyHostToDevice, c->stream));
     const int *tok_d = (const int *)(d + o_tok), *pos_d = (const int *)(d + o_pos), *sel_d = (const int *)(d + o_sel);
@@ -885,9 +889,9 @@ static int fw_pass(RqCtx *c, Pass *P, float *out) {
                                  kc_d + (size_t)l * n, vc_d + (size_t)l * n, kvt_d, grp == 5, nqm, c->part,
                                  c->pstride, s));
             else
-                KCHK(gw_k_attn_part((const Item *)items_d + off, gcnt[grp], gnq[grp], c->qkv, c->ldqkv, nh, nkv, hd,
+                KCHK(gw_k_attn_part((const Item *)items_d + off, gcnt[grp], c->qkv, c->ldqkv, nh, nkv, hd,
                                     m->att_scale, pos_d, kc_d + (size_t)l * n, vc_d + (size_t)l * n, c->part, c->pstride,
-                                    grp >> 1, s));
+                                    grp >> 1, !(grp & 1), s));
         }
         if (fused) {
             if (nbmax <= GW_GV_NBMAX) {

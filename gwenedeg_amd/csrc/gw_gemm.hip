@@ -1812,7 +1812,7 @@ void gw_take_launch_events(hipEvent_t *a, hipEvent_t *b) {
 
 static int g_tile_rows = 0; // gw_matmul_tile_rows
 
-static int gemm_cus(void) { // the device's compute units
+int gw_device_cus(void) { // the device's compute units
     static int cus = 0;
     if (!cus) {
         int dev = 0;
@@ -1861,7 +1861,7 @@ static int q8l_width(int N, int M, int K) {
     //             4,096 x 4,096 48.8 / 44.1 / 42.5; 4,096 x 12,288 133 / 122 / 119
     //   256 rows: 24,576 x 4,096 123 / 109 / 109; 12,288 x 4,096 62.9 / 66.2 / 55.1; 4,096 x 12,288 91.2 / 122 / 88.8
     if (g_q8_lds) return g_q8_lds == 2 ? 128 : g_q8_lds == 3 ? 64 : g_q8_lds >= 4 ? 12 + g_q8_lds : 0;
-    const size_t cus = (size_t)gemm_cus(), mt = (size_t)((M + 63) / 64);
+    const size_t cus = (size_t)gw_device_cus(), mt = (size_t)((M + 63) / 64);
     const size_t t32 = (size_t)((N + 31) / 32) * ((M + 31) / 32);
     if (t32 <= cus && K % 512 == 0) return 20;
     if (t32 * 2 <= 3 * cus) return 18;
@@ -1945,7 +1945,7 @@ int gw_k_matmul(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int 
     if (w->type == GW_Q8_0 && mode == 0 && (g_q8_batch == 2 ? M >= 2 : g_q8_batch == 1 ? M > GW_GEMV_MAX_ROWS : q8_gemm_rows(w, M))) {
         hipEvent_t e0, e1;
         gw_take_launch_events(&e0, &e1);
-        const int cus = gemm_cus(), nt = (w->rows + GN - 1) / GN;
+        const int cus = gw_device_cus(), nt = (w->rows + GN - 1) / GN;
         const bool g64 = g_tile_rows ? g_tile_rows == 64 : (size_t)nt * ((M + 63) / 64) >= (size_t)4 * cus; // (64-row tiles: enough for several waves per SIMD)
         // (full stages, and every buffer offset inside 2^31: the descriptor-based kernel)
         const bool full = w->cols % GKB == 0 && (size_t)(M + 64) * ldx < ((size_t)1 << 31) && (size_t)GN * w->cols < ((size_t)1 << 31);
@@ -1986,7 +1986,7 @@ int gw_k_matmul(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int 
     if (GW_IS_KQ(w->type) && M > 8 && (g_tile_rows || (size_t)((w->rows + GN - 1) / GN) * ((M + 31) / 32) >= 64)) {
         hipEvent_t e0, e1;
         gw_take_launch_events(&e0, &e1);
-        const int cus = gemm_cus(), nt = (w->rows + GN - 1) / GN;
+        const int cus = gw_device_cus(), nt = (w->rows + GN - 1) / GN;
         const bool g64 = g_tile_rows ? g_tile_rows == 64 : (size_t)nt * ((M + 63) / 64) >= (size_t)4 * cus;
         const dim3 grid(nt, g64 ? (M + 63) / 64 : (M + 31) / 32);
 #define KQ_L(TT, GG) hipExtLaunchKernelGGL((k_gemm_kq<TT, GG>), grid, dim3(256), 0, s, e0, e1, 0, (const uint8_t *)w->blocks, \

@@ -379,10 +379,11 @@ int gw_k_attn_q(const void *items, int nitems, const float *qkv, int ldqkv, int 
                 hipStream_t s);
 /* the rows of quantized caches: o = D H o' / hd from the combined attention att (n rows of nh hd), quantized into aq / as */
 int gw_k_unrot_quant(const float *att, int n, int nh, int hd, const int *kvt, int8_t *aq, float *as, int ldq, hipStream_t s);
-int gw_k_attn_part(const void *items, int nitems, int nq_max, const float *qkv, int ldqkv, int nh, int nkv, int hd, float scale,
-                   const int *pos, uint16_t *const *kc, uint16_t *const *vc, float *part, int pstride, int kbf, hipStream_t s);
+int gw_k_attn_part(const void *items, int nitems, const float *qkv, int ldqkv, int nh, int nkv, int hd, float scale,
+                   const int *pos, uint16_t *const *kc, uint16_t *const *vc, float *part, int pstride, int kbf, int narrow, hipStream_t s);
 /* the one-row pass's attention with its QK-norm, RoPE and K / V store (hd 32, 64 or 128; pos: the row's position;
  * kl / vl: its sequence's K / V cache of the layer) */
+int gw_device_cus(void);
 int gw_k_attn_decode(const float *qkv, int nh, int nkv, int hd, float scale, const float *qn, const float *kn, const float *rope,
                      int pos, uint16_t *kl, uint16_t *vl, float *part, int pstride, int kbf, hipStream_t s);
 /* the rows' attention from their key blocks' partials, quantized for wo (nbmax: the most key blocks of any row) */

@@ -20,6 +20,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_fp16.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "gw_internal.h"
 
@@ -612,346 +613,482 @@ __global__ __launch_bounds__(AQ_T) void k_attn_q(const int4 *__restrict__ items,
 #undef AQ_BODY
 }
 
-// One block of 1024 threads per item (first row r0, rows nr of one sequence at consecutive positions, kv head g, key
-// block kb): the partial result of block kb (forward.c:1346-1403 with ml) for each of the nq = nr * kv_mul query vectors
+// One block of 4 waves per item (first row r0, rows nr of one sequence at consecutive positions, kv head g, key block
+// kb): the partial result of block kb (forward.c:1346-1403 with ml) for each of the nq = nr * kv_mul <= 16 query vectors
 // that reach it: part[(row * nh + h) * pstride + kb * (hd + 2)] = o[hd] (unnormalized), m, l. Vector v = (row
-// r0 + v / kv_mul, head g * kv_mul + v % kv_mul) over positions 0..pos(row). Steps:
-//   stage: the block's K and V tiles (16-byte loads, all issued before any LDS write) and the query vectors into LDS;
-//     K rows padded by 32 bytes per 32 dims, so the 4 chunks of a position read different banks
-//   scores: lane (position p, chunk c): the fma chain over dims 32c .. 32c + 31 of every vector; the 4 chunks of a
-//     position are neighbouring lanes, added in order (a = c0 + c1 + c2 + c3, left to right), times scale
-//   softmax: one wave per vector: m = max, e = exp_att(s - m), l = 16 lane chains + the tree
-//   o: lane (vector, dim pair): the fma chains over the positions in order, V from LDS (NQ = 16: its own buffer,
-//     staged with K; else the K buffer, rewritten once the scores are done: a block's LDS stays under half a CU's)
-// hd <= 128 (hd % 32 == 0), nq <= 16.
-// a0..a7 += (q0..q7 of lane N of this lane's 16-lane row) * k: v_fmac_f32_dpp with row_newbcast, the broadcast folded
-// into the fma (one rounding, as __builtin_fmaf; the compiler does not fold a separate DPP move into v_fmac). A VALU
-// write of a DPP source needs 2 wait states before the read: the s_nop, whatever the compiler placed before the block
-// (not volatile: the compiler schedules the K reads around the blocks)
-template <int N>
-__device__ __forceinline__ void fmac8_row(float &a0, float &a1, float &a2, float &a3, float &a4, float &a5, float &a6, float &a7,
-                                          float q0, float q1, float q2, float q3, float q4, float q5, float q6, float q7, float k) {
-    asm("s_nop 1\n\t"
-                 "v_fmac_f32_dpp %0, %8, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
-                 "v_fmac_f32_dpp %1, %9, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
-                 "v_fmac_f32_dpp %2, %10, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
-                 "v_fmac_f32_dpp %3, %11, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
-                 "v_fmac_f32_dpp %4, %12, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
-                 "v_fmac_f32_dpp %5, %13, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
-                 "v_fmac_f32_dpp %6, %14, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
-                 "v_fmac_f32_dpp %7, %15, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf"
-                 : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6), "+v"(a7)
-                 : "v"(q0), "v"(q1), "v"(q2), "v"(q3), "v"(q4), "v"(q5), "v"(q6), "v"(q7), "v"(k), "n"(N));
+// r0 + v / kv_mul, head g * kv_mul + v % kv_mul) over positions 0..pos(row).
+// The fma chains run on the matrix cores: v_mfma_f32_16x16x4_f32 is four fmas in k order, each rounded once and with
+// denormals flushed as the VALU's in this build (a probe of a million chains over six ranges of values, denormals among
+// them, found every result equal), at twice the VALU's rate and without its operand broadcasts. What bounds an item is
+// those MFMAs (2 x 128 per wave at 32 cycles: 3.4 us per CU and item at 2.4 GHz).
+//   scores: wave w takes positions 64 w ..; A = K (row i of MFMA u: position 64 w + 4 i + u, a lane's 8 bytes of a dim
+//     are the rows of 4 MFMAs; k: 4 consecutive dims), B = the vectors: 8 MFMAs per chunk of 32 dims, the chunks
+//     added in order, times scale. A lane then holds 16 consecutive positions of one vector
+//   softmax: m by lane shuffles and one LDS exchange between the waves, e = exp_att(s - m) into LDS by position mod 4
+//   o: wave w takes dims 32 w ..; A = e (k: 4 consecutive positions, a lane reads its 4 steps' values as one float4),
+//     B = V (a lane's dword of a position: 2 dims, one MFMA each): the fma chains over the positions in order. l (16
+//     lane chains over p mod 16 + the tree): a lane's A values are 4 of its vector's chains, in order (wave 0)
+// K and V go from memory to registers (no LDS copy: each value is one operand of one lane): every K load of a wave is
+// issued at the top, V 16 steps ahead; V rows past the item's last position read 0 (the descriptor's range).
+// The fp32 MFMAs issue through the VALU's pipe (a probe: 32.7 cycles each alone, 40.5 with one conversion between two,
+// 4 more for every further VALU instruction), so what is left is the conversions and the softmax.
+// Measured against the LDS-staged kernel with the chains on the VALU, us per launch: 512 prompt rows behind 8,192
+// positions (33.8 k items) 2332 -> 744, a 512-row prompt's chunks 240 -> 83, 464 prompt rows of a mixed pass 193 -> 70
+#define ATM_SEG 68 // floats per (position mod 4, vector) segment of e: 64 values, segments 4 banks apart
+typedef float atm_f4 __attribute__((ext_vector_type(4)));
+template <bool KB>
+__device__ __forceinline__ float atm_val(uint32_t w, int hi) { // a 16-bit cache value of a word, as fp32 (exact)
+    if (KB) return __uint_as_float(hi ? w & 0xffff0000u : w << 16);
+    return h2f((uint16_t)(hi ? w >> 16 : w & 0xffffu));
+}
+// a lane's K load: one dim of 4 positions of a tile (f16: 8 bytes; bf16: the dim pair's 16 bytes, of which the words
+// of dim parity `quad & 1` are packed when used)
+template <bool KB>
+struct AtmK {
+    uint2 x;
+    template <int AUX = 0> __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int o) {
+        x = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, AUX));
+    }
+    __device__ __forceinline__ void words(uint32_t (&k)[2], int) const { k[0] = x.x, k[1] = x.y; }
+};
+template <>
+struct AtmK<true> {
+    uint4 x;
+    template <int AUX = 0> __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int o) {
+        x = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, AUX));
+    }
+    __device__ __forceinline__ void words(uint32_t (&k)[2], int quad) const {
+        const uint32_t sel = quad & 1 ? 0x07060302u : 0x05040100u;
+        k[0] = __builtin_amdgcn_perm(x.y, x.x, sel), k[1] = __builtin_amdgcn_perm(x.w, x.z, sel);
+    }
+};
+template <bool KB> // byte offset of positions 4 (i16 % 4) .. of dim quad in a tile (tiles: kv_k_at)
+__device__ __forceinline__ int atm_koff(int i16, int quad) {
+    return KB ? (quad >> 1) * 64 + (i16 & 3) * 16 : quad * 32 + (i16 & 3) * 8;
 }
 
-#define ATT_NQ 16
-#define ATT_HDMAX 128
-#define ATT_TH 1024
-#define ATT_KROW 1056                   // LDS bytes of 32 K dims of a tile (32 x 32 + 32 padding)
-#define ATT_KTILE (4 * ATT_KROW)        // LDS bytes of a K tile (hd <= 128)
-#define ATT_QC 36                       // LDS floats per 32-dim chunk of a query vector (32 + 4 padding)
-#define ATT_QS (4 * ATT_QC)             // LDS floats per query vector
-template <int NQ, bool KB>
-__device__ __forceinline__ void attn_part_body(const int4 *__restrict__ items, const float *__restrict__ qkv, int ldqkv, int nh,
-                                               int nkv, int hd, float scale, const int *__restrict__ pos,
-                                               uint16_t *const *__restrict__ kc, uint16_t *const *__restrict__ vc,
-                                               float *__restrict__ part, int pstride) {
-    // V staged in its own LDS buffer for NQ = 16 (prefill row blocks), else into the K buffer once the scores are done
-    // (the block's LDS stays under half a CU's: two blocks per CU); its loads are issued with K's either way.
-    // One LDS block: the query vectors, scores and lengths first (below 64 KiB, so every read of them is a base
-    // register plus an immediate offset), then the K tiles, then (NQ = 16) V. V rows at a fixed 256-byte stride,
-    // whatever hd: the o chains' reads are immediate offsets from one pointer. Up to 4 vectors (SE), the exponentials
-    // go to their own array E, written by all 16 waves, and the sums l are added while the o chains run
-    constexpr bool VL = NQ == 16, SE = NQ <= 4, DQ = NQ >= 8;
-    constexpr int QS_B = NQ * ATT_QS * 4, S_B = NQ * ATT_P * 4, E_B = SE ? S_B : 0;
-    constexpr int KS_OFF = (QS_B + S_B + E_B + NQ * 4 + 15) & ~15;
-    __shared__ __align__(16) uint8_t lds[KS_OFF + 16 * ATT_KTILE + (VL ? ATT_P * 2 * ATT_HDMAX : 0)];
-    float *const qs = (float *)lds;
-    float (*const S)[ATT_P] = (float (*)[ATT_P])(lds + QS_B);
-    float (*const E)[ATT_P] = (float (*)[ATT_P])(lds + QS_B + (SE ? S_B : 0)); // (the exponentials; S itself otherwise)
-    int *const np = (int *)(lds + QS_B + S_B + E_B);
-    uint8_t *const ks = lds + KS_OFF;
-    uint8_t *const vs = lds + KS_OFF + 16 * ATT_KTILE; // (VL only)
-    static_assert(QS_B + S_B + E_B + NQ * 4 <= 65536, "scores below 64 KiB");
-    static_assert(!SE || 2 * sizeof(lds) <= 160 * 1024, "two blocks per CU");
-    static_assert(16 * ATT_KTILE >= ATT_P * 2 * ATT_HDMAX, "V rows at 256 bytes fit the K buffer");
-    int4 it = items[blockIdx.x];
-    int r0 = it.x, nr = it.y, g = it.z, kb = it.w, kv_mul = nh / nkv, nq = nr * kv_mul, t = threadIdx.x;
-    // (x / nchk = x vmg >> 16 and x / kv_mul = x kmg >> 16 for the x < 2^10 they divide here)
-    const int TB = 32 * hd, nchk = hd / 32, vmg = (65536 + nchk - 1) / nchk, kmg = (65536 + kv_mul - 1) / kv_mul;
-    const uint8_t *K = (const uint8_t *)(kc[r0] + ((size_t)kb * nkv + g) * ATT_P * hd);
-    const uint8_t *V = (const uint8_t *)(vc[r0] + ((size_t)kb * nkv + g) * ATT_P * hd);
-    int nmx = pos[r0 + nr - 1] + 1 - kb * ATT_P;
-    nmx = nmx < ATT_P ? nmx : ATT_P;
-    int nbytes = (nmx + ATT_T - 1) / ATT_T * TB; // the tiles holding positions < nmx
-    // staging of K and V: 16 bytes per thread and round, up to 4 rounds (hd <= 128), loads issued before any use
-    uint4 k0, k1, k2, k3, v0, v1, v2, v3;
-#define ATT_LD(k, KR, VR)                                                                                                \
-    if ((t + ATT_TH * k) * 16 < nbytes) {                                                                            \
-        KR = *(const uint4 *)(K + (t + ATT_TH * k) * 16);                                                             \
-        VR = *(const uint4 *)(V + (t + ATT_TH * k) * 16);                                                             \
-    }
-    ATT_LD(0, k0, v0) ATT_LD(1, k1, v1) ATT_LD(2, k2, v2) ATT_LD(3, k3, v3)
-#undef ATT_LD
-    for (int e = t; e < NQ * ATT_QS; e += ATT_TH) { // (padding and vectors past nq: zeros)
-        int v = e / ATT_QS, c = e % ATT_QS / ATT_QC, i = e % ATT_QC, d = 32 * c + i, vr = v * kmg >> 16;
-        qs[e] = v < nq && i < 32 && d < hd ? qkv[(size_t)(r0 + vr) * ldqkv + (size_t)(g * kv_mul + v - vr * kv_mul) * hd + d] : 0.0f;
-    }
-    if (t < NQ) {
-        int n = t < nq ? pos[r0 + (t * kmg >> 16)] + 1 - kb * ATT_P : 0;
-        np[t] = n < 0 ? 0 : n < ATT_P ? n : ATT_P;
-    }
-    // (V: 16-byte piece o of the block's rows, position o / (2 hd), into that position's 256-byte LDS row)
-    auto vrow = [&](int o) __attribute__((always_inline)) -> int {
-        const int pp = (o >> 6) * vmg >> 16;
-        return pp * 2 * ATT_HDMAX + (o - pp * 64 * nchk);
-    };
-#define ATT_ST(k, KR, VR)                                                                                                \
-    if ((t + ATT_TH * k) * 16 < nbytes) {                                                                            \
-        int o = (t + ATT_TH * k) * 16, tile = ((t >> 6) + 16 * k) * vmg >> 16, w = o - tile * TB;                    \
-        *(uint4 *)(ks + tile * ATT_KTILE + (w >> 10) * ATT_KROW + (w & 1023)) = KR;                                   \
-        if (VL) *(uint4 *)(vs + vrow(o)) = VR;                                                                        \
-    }
-    ATT_ST(0, k0, v0) ATT_ST(1, k1, v1) ATT_ST(2, k2, v2) ATT_ST(3, k3, v3)
-#undef ATT_ST
-    __syncthreads();
-    // scores, 8 or 16 vectors (DQ): lane 16 c + n of wave w takes position p = 16 w + n (the wave's tile w) and chunk
-    // c; the lane holds q[v][32 c + n] and q[v][32 c + 16 + n] of every vector in registers, and dim i of the chunk's
-    // chain takes the row's lane i % 16's (a DPP broadcast inside the fma): no query reads from LDS in the chains.
-    // The chunks of position p are rows 0 .. 3 of lane n, added in order. Every lane of a wave whose tile holds a
-    // position of the block runs the chains (no lane masked: a DPP source lane must be active); lanes past the block
-    // or the head's chunks compute values never written
-    if constexpr (DQ) {
-        const int n = t & 15, c = (t >> 4) & 3, wv = __builtin_amdgcn_readfirstlane(t >> 6), p = 16 * wv + n;
-        float qa[NQ], qb[NQ], acc[NQ];
-        #pragma unroll
-        for (int v = 0; v < NQ; v++) {
-            qa[v] = qs[v * ATT_QS + c * ATT_QC + n];
-            qb[v] = qs[v * ATT_QS + c * ATT_QC + 16 + n];
-            acc[v] = 0.0f;
-        }
-        if (16 * wv < nmx) {
-            const uint8_t *kt = ks + wv * ATT_KTILE + c * ATT_KROW + (KB ? 4 : 2) * n;
-#define ATT_DQ(I, KF)                                                                                                   \
-            {                                                                                                           \
-                const float kf_ = (KF);                                                                                 \
-                const float *qq = (I) < 16 ? qa : qb;                                                                   \
-                fmac8_row<(I) & 15>(acc[0], acc[1], acc[2], acc[3], acc[4], acc[5], acc[6], acc[7], qq[0], qq[1], qq[2],  \
-                                    qq[3], qq[4], qq[5], qq[6], qq[7], kf_);                                            \
-                if constexpr (NQ > 8)                                                                                   \
-                    fmac8_row<(I) & 15>(acc[8], acc[9], acc[10], acc[11], acc[12], acc[13], acc[14], acc[15], qq[8],      \
-                                        qq[9], qq[10], qq[11], qq[12], qq[13], qq[14], qq[15], kf_);                    \
-            }
-            if constexpr (KB) { // (dims i, i + 1 of position p: one word at i 32 + 4 p of the chunk row, i even)
-#define ATT_DQ2(I)                                                                                                      \
-                {                                                                                                       \
-                    const uint32_t w_ = *(const uint32_t *)(kt + (I) * 32);                                             \
-                    ATT_DQ(I, bf2f(w_ & 0xffffu))                                                                       \
-                    ATT_DQ((I) + 1, bf2f(w_ >> 16))                                                                     \
-                }
-                ATT_DQ2(0) ATT_DQ2(2) ATT_DQ2(4) ATT_DQ2(6) ATT_DQ2(8) ATT_DQ2(10) ATT_DQ2(12) ATT_DQ2(14)
-                ATT_DQ2(16) ATT_DQ2(18) ATT_DQ2(20) ATT_DQ2(22) ATT_DQ2(24) ATT_DQ2(26) ATT_DQ2(28) ATT_DQ2(30)
-#undef ATT_DQ2
-            } else {
-#define ATT_DQ1(I) ATT_DQ(I, h2f(*(const uint16_t *)(kt + (I) * 32)))
-                ATT_DQ1(0) ATT_DQ1(1) ATT_DQ1(2) ATT_DQ1(3) ATT_DQ1(4) ATT_DQ1(5) ATT_DQ1(6) ATT_DQ1(7)
-                ATT_DQ1(8) ATT_DQ1(9) ATT_DQ1(10) ATT_DQ1(11) ATT_DQ1(12) ATT_DQ1(13) ATT_DQ1(14) ATT_DQ1(15)
-                ATT_DQ1(16) ATT_DQ1(17) ATT_DQ1(18) ATT_DQ1(19) ATT_DQ1(20) ATT_DQ1(21) ATT_DQ1(22) ATT_DQ1(23)
-                ATT_DQ1(24) ATT_DQ1(25) ATT_DQ1(26) ATT_DQ1(27) ATT_DQ1(28) ATT_DQ1(29) ATT_DQ1(30) ATT_DQ1(31)
-#undef ATT_DQ1
-            }
-#undef ATT_DQ
-        }
-        #pragma unroll
-        for (int v = 0; v < NQ; v++) {
-            float c1 = __shfl_down(acc[v], 16), c2 = __shfl_down(acc[v], 32), c3 = __shfl_down(acc[v], 48);
-            float a = acc[v];
-            if (nchk > 1) a = a + c1;
-            if (nchk > 2) a = a + c2;
-            if (nchk > 3) a = a + c3;
-            if (c == 0 && p < nmx && v < nq) S[v][p] = a * scale;
-        }
-    } else { // scores, up to 4 vectors: lane (position p, chunk c), all NQ vectors (no per-vector branches in the chain)
-        int p = t >> 2, c = t & 3;
-        const uint8_t *kt = ks + (p / ATT_T) * ATT_KTILE + c * ATT_KROW + (p % ATT_T) * 2;
-        const float *qc = qs + c * ATT_QC;
-        float acc[NQ];
-        #pragma unroll
-        for (int v = 0; v < NQ; v++) acc[v] = 0.0f;
-        if (p < nmx && c < nchk) {
-            for (int i = 0; i < 32; i += 4) {
-                float k[4];
-                if (KB) { // (dims i, i + 1 of position p in one word at i 32 + 4 p of the chunk row; i + 2, i + 3 below)
-                    const uint8_t *kw = kt + (p % ATT_T) * 2;
-                    const uint32_t d0 = *(const uint32_t *)(kw + i * 32), d1 = *(const uint32_t *)(kw + (i + 2) * 32);
-                    k[0] = bf2f(d0 & 0xffffu), k[1] = bf2f(d0 >> 16), k[2] = bf2f(d1 & 0xffffu), k[3] = bf2f(d1 >> 16);
-                } else {
-                    #pragma unroll
-                    for (int u = 0; u < 4; u++) k[u] = h2f(*(const uint16_t *)(kt + (i + u) * 32));
-                }
-                float4 q4[NQ];
-                #pragma unroll
-                for (int v = 0; v < NQ; v++) q4[v] = *(const float4 *)(qc + v * ATT_QS + i);
-                #pragma unroll
-                for (int v = 0; v < NQ; v++) {
-                    acc[v] = __builtin_fmaf(q4[v].x, k[0], acc[v]);
-                    acc[v] = __builtin_fmaf(q4[v].y, k[1], acc[v]);
-                    acc[v] = __builtin_fmaf(q4[v].z, k[2], acc[v]);
-                    acc[v] = __builtin_fmaf(q4[v].w, k[3], acc[v]);
-                }
-            }
-        }
-        #pragma unroll
-        for (int v = 0; v < NQ; v++) {
-            float c1 = quad_lane<1>(acc[v]), c2 = quad_lane<2>(acc[v]), c3 = quad_lane<3>(acc[v]); // (chunks of lane c = 0)
-            float a = acc[v];
-            if (nchk > 1) a = a + c1;
-            if (nchk > 2) a = a + c2;
-            if (nchk > 3) a = a + c3;
-            if (c == 0 && p < nmx && v < nq) S[v][p] = a * scale;
-        }
-    }
-    __syncthreads();
-    if (!VL) { // V into the K buffer (its readers are done), position p's row at p 256 bytes
-#define ATT_SV(k, VR)                                                                                                    \
-        if ((t + ATT_TH * k) * 16 < nbytes) *(uint4 *)(ks + vrow((t + ATT_TH * k) * 16)) = VR;
-        ATT_SV(0, v0) ATT_SV(1, v1) ATT_SV(2, v2) ATT_SV(3, v3)
-#undef ATT_SV
-    }
-    // (the wave and a wave's vector length as uniform values: scalar loop bounds, no exec-masked loops)
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
-    // (a vector's part of block kb: m, l after its hd values o)
-    auto mlp = [&](int v) __attribute__((always_inline)) -> float * {
-        return part + ((size_t)(r0 + v / kv_mul) * nh + g * kv_mul + v % kv_mul) * pstride + (size_t)kb * (hd + 2) + hd;
-    };
-    if (SE) { // softmax: wave w takes vector w & 3 (its max over the block, each of its 4 waves alike), positions
-              // 64 (w >> 2) + lane: E = exp_att(s - m); l is added after the barrier, beside the o chains
-        const int v = wave & 3, p = 64 * (wave >> 2) + lane;
-        if (v < nq && np[v] > 0) {
-            const int n = np[v];
-            float m = -3.402823466e38f;
-            for (int q = lane; q < n; q += 64) m = fmaxf(m, S[v][q]);
-            m = wave_max(m);
-            if (p < n) E[v][p] = exp_att(S[v][p] - m);
-            if (wave < 4 && lane == 0) mlp(v)[0] = m;
-        }
-    } else if (wave < nq && np[wave] > 0) { // softmax: wave v takes vector v
-        int v = wave, n = np[v];
-        float m = -3.402823466e38f;
-        for (int p = lane; p < n; p += 64) m = fmaxf(m, S[v][p]);
-        m = wave_max(m);
-        for (int p = lane; p < n; p += 64) S[v][p] = exp_att(S[v][p] - m);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        float s = 0.0f;
-        if (lane < 16) {
-            int p = lane;
-            for (; p + 48 < n; p += 64) {
-                float e0 = S[v][p], e1 = S[v][p + 16], e2 = S[v][p + 32], e3 = S[v][p + 48];
-                s = s + e0;
-                s = s + e1;
-                s = s + e2;
-                s = s + e3;
-            }
-            for (; p < n; p += 16) s = s + S[v][p];
-        }
-        for (int w = 8; w >= 1; w >>= 1) {
-            float o = __shfl_down(s, w);
-            s = s + o;
-        }
-        if (lane == 0) {
-            float *ml = mlp(v);
-            ml[0] = m;
-            ml[1] = s;
-        }
-    }
-    __syncthreads();
-    if (SE && wave >= 4 && wave < 8 && wave - 4 < nq && np[wave - 4] > 0) { // l of vector wave - 4: 16 lane chains
-        const int v = wave - 4, n = np[v];                                  // over p = lane (mod 16), then the tree
-        float s = 0.0f;
-        if (lane < 16) {
-            int p = lane;
-            for (; p + 48 < n; p += 64) {
-                float e0 = E[v][p], e1 = E[v][p + 16], e2 = E[v][p + 32], e3 = E[v][p + 48];
-                s = s + e0;
-                s = s + e1;
-                s = s + e2;
-                s = s + e3;
-            }
-            for (; p < n; p += 16) s = s + E[v][p];
-        }
-        for (int w = 8; w >= 1; w >>= 1) {
-            float o = __shfl_down(s, w);
-            s = s + o;
-        }
-        if (lane == 0) mlp(v)[1] = s;
-    }
-    // o: lane (vector v = wave, dim pair d2): the chains over the positions in order, V pairs from LDS, two register
-    // sets of PB positions' loads per step
-    {
-        int v = wave, d2 = lane, i0 = 2 * d2;
-        const int n = v < NQ ? __builtin_amdgcn_readfirstlane(np[v < NQ ? v : 0]) : 0;
-        if (v < nq && i0 < hd && n > 0) {
-            int p = 0;
-            float o0 = 0.0f, o1 = 0.0f;
-            // (the V rows' byte offset opaque to the compiler: one base register with immediate offsets, not a sum
-            // folded into every read past 64 KiB (NQ = 16: V lies above the K tiles))
-            int vo = (int)((VL ? vs : ks) - lds) + i0 * 2;
-            asm volatile("" : "+v"(vo));
-            const uint32_t *vb = (const uint32_t *)(lds + vo);
-            constexpr int rs = ATT_HDMAX / 2; // (uint32 words per position's LDS row)
-            constexpr int PB = VL ? 16 : 8; // (8: 64 registers, two blocks per CU)
-            uint32_t va[PB], vbb[PB];
-            float ea[PB], eb[PB];
-            auto ld = [&](uint32_t (&vv)[PB], float (&ee)[PB], int q0) {
-                #pragma unroll
-                for (int u = 0; u < PB; u++) {
-                    vv[u] = vb[(q0 + u) * rs];
-                    ee[u] = E[v][q0 + u];
-                }
-            };
-            auto fold = [&](const uint32_t (&vv)[PB], const float (&ee)[PB]) {
-                #pragma unroll
-                for (int u = 0; u < PB; u++) {
-                    o0 = __builtin_fmaf(ee[u], KB ? bf2f(vv[u] & 0xffffu) : h2f((uint16_t)(vv[u] & 0xffff)), o0);
-                    o1 = __builtin_fmaf(ee[u], KB ? bf2f(vv[u] >> 16) : h2f((uint16_t)(vv[u] >> 16)), o1);
-                }
-            };
-            // (each step loads both sets, then folds them: no register set carried across steps, whose copies had
-            // cost a fifth of the loop's instructions; the block's other waves cover the loads' latency)
-            for (; p + 2 * PB <= n; p += 2 * PB) {
-                ld(va, ea, p);
-                ld(vbb, eb, p + PB);
-                fold(va, ea);
-                fold(vbb, eb);
-            }
-            if (p + PB <= n) {
-                ld(va, ea, p);
-                fold(va, ea);
-                p += PB;
-            }
-            for (; p < n; p++) {
-                uint32_t vv = vb[p * rs];
-                float e = E[v][p];
-                o0 = __builtin_fmaf(e, KB ? bf2f(vv & 0xffffu) : h2f((uint16_t)(vv & 0xffff)), o0);
-                o1 = __builtin_fmaf(e, KB ? bf2f(vv >> 16) : h2f((uint16_t)(vv >> 16)), o1);
-            }
-            int row = r0 + v / kv_mul, h = g * kv_mul + v % kv_mul;
-            float *o = part + ((size_t)row * nh + h) * pstride + (size_t)kb * (hd + 2);
-            // (a V word holds dims i0, i0 + 1; in a bf16 row, dims 32 c + l and 32 c + 16 + l, d2 = 16 c + l)
-            const int da = KB ? 32 * (d2 >> 4) + (d2 & 15) : i0, db = KB ? da + 16 : i0 + 1;
-            o[da] = o0;
-            o[db] = o1;
-        }
-    }
-}
-
-template <int NQ, bool KB>
-__global__ __launch_bounds__(ATT_TH, NQ <= 4 ? 8 : 4) void k_attn_part(const int4 *__restrict__ items, const float *__restrict__ qkv, int ldqkv,
-                                                      int nh, int nkv, int hd, float scale, const int *__restrict__ pos,
+template <int HD, bool KB>
+__global__ __launch_bounds__(256, 3) void k_attn_part(const int4 *__restrict__ items, const float *__restrict__ qkv, int ldqkv,
+                                                      int nh, int nkv, float scale, const int *__restrict__ pos,
                                                       uint16_t *const *__restrict__ kc, uint16_t *const *__restrict__ vc,
                                                       float *__restrict__ part, int pstride) {
-    attn_part_body<NQ, KB>(items, qkv, ldqkv, nh, nkv, hd, scale, pos, kc, vc, part, pstride);
+    constexpr int NCH = HD / 32, QS = HD + 4; // (chunks, LDS floats per vector)
+    __shared__ __align__(16) float qs[16 * QS];
+    __shared__ __align__(16) float es[64 * ATM_SEG];
+    __shared__ float red[4][16];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), i16 = lane & 15, quad = lane >> 4;
+    const int4 it = items[blockIdx.x];
+    const int r0 = it.x, nr = it.y, g = it.z, kb = it.w, kv_mul = nh / nkv, nq = nr * kv_mul;
+    const int kmg = (65536 + kv_mul - 1) / kv_mul; // (x / kv_mul = x kmg >> 16 for the x < 16 it divides here)
+    int nmx = pos[r0 + nr - 1] + 1 - kb * ATT_P, nmn = pos[r0] + 1 - kb * ATT_P;
+    nmx = nmx < ATT_P ? nmx : ATT_P;
+    nmn = nmn < 0 ? 0 : nmn < ATT_P ? nmn : ATT_P; // (the first row's positions in the block: the fewest of the item)
+    // the query vectors' loads before the cache's (loads complete in order)
+    constexpr int NQL = (4 * HD + 255) / 256;
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)(qkv + (size_t)r0 * ldqkv), (short)0, nr * ldqkv * 4, GW_RSRC_DW3);
+    float4 qx[NQL];
+    #pragma unroll
+    for (int i = 0; i < NQL; i++) {
+        const int e = t + 256 * i, v = e / (HD / 4), vr = v * kmg >> 16; // (past nq: past the descriptor, 0)
+        const int o = (vr * ldqkv + (g * kv_mul + v - vr * kv_mul) * HD + 4 * (e % (HD / 4))) * 4;
+        qx[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rq, v < nq ? o : nr * ldqkv * 4, 0, 0));
+    }
+    const int npos = pos[r0 + ((i16 < nq ? i16 : 0) * kmg >> 16)];
+    __builtin_amdgcn_sched_barrier(0);
+    const uint16_t *K = kc[r0] + ((size_t)kb * nkv + g) * ATT_P * HD, *V = vc[r0] + ((size_t)kb * nkv + g) * ATT_P * HD;
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)K, (short)0, ((nmx + ATT_T - 1) & ~(ATT_T - 1)) * HD * 2, GW_RSRC_DW3);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)V, (short)0, nmx * HD * 2, GW_RSRC_DW3);
+    AtmK<KB> kr[8 * NCH]; // dims 4 s + quad of positions 64 w + 4 i16 + (0 .. 3)
+    const int ko = (4 * w + (i16 >> 2)) * 32 * HD + atm_koff<KB>(i16, quad);
+    auto kload = [&](int c) __attribute__((always_inline)) {
+        #pragma unroll
+        for (int s = 8 * c; s < 8 * c + 8; s++) kr[s].load(rk, ko + 128 * s);
+    };
+    const bool kin = 64 * w < nmx; // (uniform: the wave's positions reach into the block)
+    #pragma unroll // (unconditional: past the block's tiles they read 0)
+    for (int c = 0; c < (KB && NCH > 2 ? 2 : NCH); c++) kload(c);
+    // the query vectors into LDS (past nq: zeros)
+    #pragma unroll
+    for (int i = 0; i < NQL; i++) {
+        const int e = t + 256 * i, v = e / (HD / 4);
+        if (NQL * 256 == 4 * HD || e < 4 * HD)
+            *(float4 *)(qs + v * QS + 4 * (e % (HD / 4))) = qx[i];
+    }
+    // this lane's vector (i16): its positions in the block
+    int n = i16 < nq ? npos + 1 - kb * ATT_P : 0;
+    n = n < 0 ? 0 : n < ATT_P ? n : ATT_P;
+    __syncthreads();
+    // scores: sc[u][r] of position p0 + 4 r + u
+    typedef atm_f4 f4;
+    const int p0 = 64 * w + 16 * quad;
+    f4 sc[4] = {};
+    if (kin) {
+        #pragma unroll
+        for (int c = 0; c < NCH; c++) {
+            float qr[8];
+            #pragma unroll
+            for (int s = 0; s < 8; s++) qr[s] = qs[i16 * QS + 32 * c + 4 * s + quad];
+            f4 a[4] = {};
+            #pragma unroll
+            for (int s = 0; s < 8; s++) {
+                uint32_t k[2];
+                kr[8 * c + s].words(k, quad);
+                #pragma unroll
+                for (int u = 0; u < 4; u++) a[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(atm_val<KB>(k[u >> 1], u & 1), qr[s], a[u], 0, 0, 0);
+            }
+            if (KB && c + 2 < NCH) kload(c + 2);
+            #pragma unroll
+            for (int u = 0; u < 4; u++) sc[u] = c ? sc[u] + a[u] : a[u];
+        }
+    }
+    // V: wave w's dims, a dword of positions 4 s + quad (16 steps of 4 positions per set; past nmx: 0, the whole offset in
+    // the per-lane operand, which the descriptor's range check covers)
+    const int vo = NCH == 4 || w < NCH ? quad * HD * 2 + 64 * w + 4 * i16 : ATT_P * HD * 2;
+    uint32_t va[16], vb[16];
+    auto vload = [&](uint32_t (&v)[16], int c) __attribute__((always_inline)) {
+        #pragma unroll
+        for (int s = 0; s < 16; s++)
+            v[s] = __builtin_amdgcn_raw_buffer_load_b32(rv, vo + c * 128 * HD + s * 8 * HD, 0, 0);
+    };
+    vload(va, 0);
+    // softmax
+    float m = -3.402823466e38f;
+    #pragma unroll
+    for (int u = 0; u < 4; u++)
+        #pragma unroll
+        for (int r = 0; r < 4; r++) {
+            sc[u][r] = sc[u][r] * scale;
+            if (p0 + 4 * r + u < n) m = fmaxf(m, sc[u][r]);
+        }
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    if (quad == 0) red[w][i16] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0][i16], red[1][i16]), fmaxf(red[2][i16], red[3][i16]));
+    #pragma unroll
+    for (int u = 0; u < 4; u++) { // (positions p0 + 4 r + u: value (p0 + 4 r) / 4 of segment u)
+        f4 e;
+        #pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float x = exp_att(sc[u][r] - m);
+            e[r] = p0 + 4 * r + u < n ? x : 0.0f;
+        }
+        *(f4 *)(es + (u * 16 + i16) * ATM_SEG + (p0 >> 2)) = e;
+    }
+    __syncthreads();
+    if (NCH < 4 && w >= NCH) return;
+    // o: D row (vector) 4 quad + r, column i16
+    f4 o0 = {}, o1 = {}, ls = {};
+    const float *er = es + (quad * 16 + i16) * ATM_SEG;
+    const int nc = (nmx + 63) >> 6;
+    auto fold = [&](const uint32_t (&v)[16], int c, auto diag) __attribute__((always_inline)) {
+        f4 e[4];
+        #pragma unroll
+        for (int k = 0; k < 4; k++) e[k] = *(const f4 *)(er + 16 * c + 4 * k);
+        if (w == 0) {
+            #pragma unroll
+            for (int k = 0; k < 4; k++) ls = ls + e[k];
+        }
+        const f4 b0 = o0, b1 = o1;
+        #pragma unroll
+        for (int s = 0; s < 16; s++) {
+            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(e[s >> 2][s & 3], atm_val<KB>(v[s], 0), o0, 0, 0, 0);
+            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(e[s >> 2][s & 3], atm_val<KB>(v[s], 1), o1, 0, 0, 0);
+        }
+        if (decltype(diag)::value && 64 * c + 64 > nmn) {
+            // positions that only the item's later rows reach: their e is 0 for the earlier rows, which adds nothing
+            // unless V is not finite (0 NaN, 0 inf). Then o is not finite either: each row folds the positions again
+            // with those past its own as 0
+            f4 z = {};
+            #pragma unroll
+            for (int r = 0; r < 4; r++) z[r] = (o0[r] - o0[r]) + (o1[r] - o1[r]); // (0, or NaN)
+            const float zz = (z[0] + z[1]) + (z[2] + z[3]);
+            if (__ballot(!(zz == 0.0f))) {
+                for (int rr = 0; rr < nr; rr++) {
+                    f4 x0 = b0, x1 = b1;
+                    const int nrow = pos[r0 + rr] + 1 - kb * ATT_P;
+                    #pragma unroll
+                    for (int s = 0; s < 16; s++) {
+                        const uint32_t x = 64 * c + 4 * s + quad < nrow ? v[s] : 0u;
+                        x0 = __builtin_amdgcn_mfma_f32_16x16x4f32(e[s >> 2][s & 3], atm_val<KB>(x, 0), x0, 0, 0, 0);
+                        x1 = __builtin_amdgcn_mfma_f32_16x16x4f32(e[s >> 2][s & 3], atm_val<KB>(x, 1), x1, 0, 0, 0);
+                    }
+                    #pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if ((4 * quad + r) * kmg >> 16 == rr) o0[r] = x0[r], o1[r] = x1[r];
+                }
+            }
+        }
+    };
+    auto chains = [&](auto diag) __attribute__((always_inline)) {
+        for (int c = 0; c < nc; c += 2) { // (loads past the block read 0, without a branch around them)
+            vload(vb, c + 1);
+            fold(va, c, diag);
+            vload(va, c + 2);
+            if (c + 1 < nc) fold(vb, c + 1, diag);
+        }
+    };
+    if (nmn < nmx) chains(std::true_type{}); // (the block of the diagonal)
+    else chains(std::false_type{});
+    // (a vector's part of block kb: hd values o, then m, l)
+    auto dst = [&](int v) __attribute__((always_inline)) -> float * {
+        const int vr = v * kmg >> 16;
+        return part + ((size_t)(r0 + vr) * nh + g * kv_mul + v - vr * kv_mul) * pstride + (size_t)kb * (HD + 2);
+    };
+    #pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int v = 4 * quad + r, nv = __shfl(n, v); // (lane v holds vector v's positions)
+        if (v < nq && nv > 0) {
+            float *o = dst(v) + 32 * w;
+            if constexpr (KB) { // (a dword of a bf16 row: dims 32 c + j and 32 c + 16 + j)
+                o[i16] = o0[r];
+                o[16 + i16] = o1[r];
+            } else {
+                *(float2 *)(o + 2 * i16) = make_float2(o0[r], o1[r]);
+            }
+        }
+    }
+    if (w == 0) { // l: ls[a] is chain 4 a + quad; the tree +8 +4 in the lane, +2 +1 between the quads
+        float l = (ls[0] + ls[2]) + (ls[1] + ls[3]);
+        l = l + __shfl_down(l, 32);
+        l = l + __shfl_down(l, 16);
+        if (quad == 0 && i16 < nq && n > 0) {
+            float *ml = dst(i16) + HD;
+            ml[0] = m;
+            ml[1] = l;
+        }
+    }
+}
+
+// Up to 4 query vectors of one row over one key block (decode rows), by 4 waves: the partial as k_attn_part's, with
+// v_mfma_f32_4x4x1_f32 (16 blocks of 4 x 4, one fma per output: no padding at 4 vectors, 8 cycles).
+//   scores (attn4_scores): wave w takes positions 64 w .., K loads as k_attn_part's (whole 128-byte lines); a 4 x 4
+//     transpose of registers against 16-lane rows (v_permlane32_swap / v_permlane16_swap) then gives row c of the wave
+//     chunk c, so a lane runs the whole chain of one chunk for 4 positions (block: 4 lanes; A: K, B: the vectors). The
+//     same transpose brings a position's 4 chunks together, added in order: a lane ends with 4 consecutive positions of
+//     vector lane % 4
+//   softmax (attn4_softmax): m by lane shuffles and one LDS exchange between the waves, e into LDS
+//   o (attn4_chains): two waves, one for the low and one for the high halves of the V rows' dwords (lane i loads dword i of
+//     each position): A = e, B = V, the chains over the positions in order. (V by 16-byte loads, transposed as K is: 64
+//     loads instead of 256, but the swaps cost 16 cycles each: 217 against 202 us on the 8 x 32,768 positions)
+//   l (attn4_l): another wave
+#define ATM4_EP 260 // floats per vector of e (256 + 4)
+#define ATM4_NT 2   // the batched rows' K / V loads are non-temporal (read once per layer)
+__device__ __forceinline__ void atm_tr4(uint32_t &a, uint32_t &b, uint32_t &c, uint32_t &d) {
+    // register i of lane row j <-> register j of lane row i (rows of 16 lanes)
+    auto x = __builtin_amdgcn_permlane32_swap(a, c, false, false);
+    a = x[0], c = x[1];
+    x = __builtin_amdgcn_permlane32_swap(b, d, false, false);
+    b = x[0], d = x[1];
+    x = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = x[0], b = x[1];
+    x = __builtin_amdgcn_permlane16_swap(c, d, false, false);
+    c = x[0], d = x[1];
+}
+template <int HD, bool KB, int NT>
+struct Attn4K { // a wave's K: dims 4 s + quad of positions 64 w + 4 i16 + (0 .. 3), s = 8 c + k (bf16: half in flight)
+    static constexpr int NCH = HD / 32;
+    AtmK<KB> kr[8 * NCH];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rk, int ko, int k) {
+        #pragma unroll
+        for (int c = 0; c < NCH; c++) kr[8 * c + k].template load<NT>(rk, ko + 128 * (8 * c + k));
+    }
+    // (unconditional: past the block's tiles, which the descriptor ends at, they read 0)
+    __device__ __forceinline__ void first(__amdgpu_buffer_rsrc_t rk, int ko) {
+        #pragma unroll
+        for (int k = 0; k < (KB ? 4 : 8); k++) load(rk, ko, k);
+    }
+};
+// sc[u]: the scaled score of position 64 w + 16 (i16 / 4) + 4 quad + u, vector lane % 4. fix(k, x): may replace words of
+// dims 4 k + j (x[j]) of chunk `quad`, positions 4 i16 + (0 .. 3)
+template <int HD, bool KB, int NT, typename F>
+__device__ __forceinline__ void attn4_scores(Attn4K<HD, KB, NT> &K, __amdgpu_buffer_rsrc_t rk, int ko, const float *qs, float scale,
+                                             float (&sc)[4], F fix) {
+    constexpr int NCH = HD / 32;
+    const int lane = threadIdx.x & 63, quad = lane >> 4;
+    atm_f4 a[4] = {};
+    #pragma unroll
+    for (int k = 0; k < 8; k++) {
+        uint32_t x[4][2];
+        #pragma unroll
+        for (int c = 0; c < 4; c++) {
+            x[c][0] = x[c][1] = 0;
+            if (c < NCH) K.kr[(c < NCH ? 8 * c : 0) + k].words(x[c], quad);
+        }
+        if (KB && k < 4) K.load(rk, ko, k + 4);
+        atm_tr4(x[0][0], x[1][0], x[2][0], x[3][0]); // (x[j]: dim 4 k + j of chunk `quad`)
+        atm_tr4(x[0][1], x[1][1], x[2][1], x[3][1]);
+        fix(k, x);
+        const atm_f4 q = *(const atm_f4 *)(qs + (lane & 3) * 128 + 32 * quad + 4 * k);
+        float kf[4][4];
+        #pragma unroll
+        for (int j = 0; j < 4; j++)
+            #pragma unroll
+            for (int u = 0; u < 4; u++) kf[j][u] = atm_val<KB>(x[j][u >> 1], u & 1);
+        __builtin_amdgcn_sched_barrier(0); // (the conversions apart from the MFMAs: each change between the two costs 4 cycles)
+        #pragma unroll
+        for (int j = 0; j < 4; j++)
+            #pragma unroll
+            for (int u = 0; u < 4; u++) a[u] = __builtin_amdgcn_mfma_f32_4x4x1f32(kf[j][u], q[j], a[u], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    #pragma unroll
+    for (int u = 0; u < 4; u++) { // (a[u][r]: chunk `quad` of position 64 w + 16 (i16 / 4) + 4 r + u)
+        uint32_t y[4];
+        #pragma unroll
+        for (int r = 0; r < 4; r++) y[r] = __float_as_uint(a[u][r]);
+        atm_tr4(y[0], y[1], y[2], y[3]);
+        float x = __uint_as_float(y[0]);
+        #pragma unroll
+        for (int c = 1; c < NCH; c++) x = x + __uint_as_float(y[c]);
+        sc[u] = x * scale;
+    }
+}
+// e of the block's n positions into es (0 past n); returns m of vector lane % 4 (two barriers, all 4 waves)
+__device__ __forceinline__ float attn4_softmax(const float (&sc)[4], int w, int p0, int n, float (*red)[4], float *es) {
+    const int lane = threadIdx.x & 63, v = lane & 3;
+    float m = -3.402823466e38f;
+    if (w < 4) {
+        #pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (p0 + u < n) m = fmaxf(m, sc[u]);
+        m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0x124, 0xF, 0xF, true))); // (row_ror:4)
+        m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0x128, 0xF, 0xF, true))); // (row_ror:8)
+        m = fmaxf(m, __shfl_xor(m, 16));
+        m = fmaxf(m, __shfl_xor(m, 32));
+        if (lane < 4) red[w][lane] = m;
+    }
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0][v], red[1][v]), fmaxf(red[2][v], red[3][v]));
+    if (w < 4) {
+        atm_f4 e;
+        #pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const float x = exp_att(sc[u] - m);
+            e[u] = p0 + u < n ? x : 0.0f;
+        }
+        *(atm_f4 *)(es + v * ATM4_EP + p0) = e;
+    }
+    __syncthreads();
+    return m;
+}
+template <int HD, int NT>
+struct Attn4V { // 16 positions of V: this lane's dword of each row
+    uint32_t x[16];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rv, int vo, int p) {
+        #pragma unroll
+        for (int s = 0; s < 16; s++) x[s] = __builtin_amdgcn_raw_buffer_load_b32(rv, vo + (p + s) * HD * 2, 0, NT);
+    }
+};
+template <int HD>
+__device__ __forceinline__ int attn4_vo() { // the lane's byte offset in a V row (lanes past the row: past the descriptor)
+    const int lane = threadIdx.x & 63;
+    return lane < HD / 2 ? 4 * lane : ATT_P * HD * 2;
+}
+// the o chains of the dims in a row dword's half HI over the n positions (e 0 past n, V 0 past its descriptor): o[r] of
+// vector r, this lane's dword. A: positions 0 .. 15, already loading
+template <int HD, bool KB, int HI, int NT>
+__device__ __forceinline__ atm_f4 attn4_chains(Attn4V<HD, NT> &A, Attn4V<HD, NT> &B, __amdgpu_buffer_rsrc_t rv, int vo, const float *es, int n) {
+    atm_f4 o = {};
+    const float *er = es + (threadIdx.x & 3) * ATM4_EP;
+    auto fold = [&](const Attn4V<HD, NT> &V, int p) __attribute__((always_inline)) {
+        atm_f4 ev[4];
+        float f[16];
+        #pragma unroll
+        for (int k = 0; k < 4; k++) ev[k] = *(const atm_f4 *)(er + p + 4 * k);
+        #pragma unroll
+        for (int s = 0; s < 16; s++) f[s] = atm_val<KB>(V.x[s], HI);
+        __builtin_amdgcn_sched_barrier(0);
+        #pragma unroll
+        for (int s = 0; s < 16; s++) o = __builtin_amdgcn_mfma_f32_4x4x1f32(ev[s >> 2][s & 3], f[s], o, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int p = 0; p < n; p += 32) {
+        B.load(rv, vo, p + 16);
+        fold(A, p);
+        A.load(rv, vo, p + 32);
+        fold(B, p + 16);
+    }
+    return o;
+}
+// l of vector quad (lanes i16 = 0): lane i16 is chain i16, then the tree
+__device__ __forceinline__ float attn4_l(const float *es) {
+    const int lane = threadIdx.x & 63;
+    const float *er = es + (lane >> 4) * ATM4_EP + (lane & 15);
+    float c[16], s = 0.0f;
+    #pragma unroll
+    for (int k = 0; k < 16; k++) c[k] = er[16 * k];
+    #pragma unroll
+    for (int k = 0; k < 16; k++) s = s + c[k];
+    s = s + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x108, 0xF, 0xF, true));
+    s = s + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x104, 0xF, 0xF, true));
+    s = s + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x102, 0xF, 0xF, true));
+    return s + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x101, 0xF, 0xF, true));
+}
+
+// dword i of a V row: its low half's dim (f16: 2 i; bf16 rows hold dims 32 c + j and 32 c + 16 + j in a dword)
+template <bool KB>
+__device__ __forceinline__ int attn4_dim(int i, int hi) { return KB ? 32 * (i >> 4) + (i & 15) + 16 * hi : 2 * i + hi; }
+
+// k_attn_part for items of one row with at most 4 query vectors. The item's arithmetic (2 us per CU) is under half of the
+// time its 128 KB take from HBM, which bounds it. 8 rows x 32,768 positions (8256 items, 1.08 GB), us: 226 LDS-staged
+// with the chains on the VALU, 214 k_attn_part, 202 here (5.4 TB/s); 32 rows x 2,048: 68 -> 56.5
+template <int HD, bool KB>
+__global__ __launch_bounds__(256, KB ? 3 : 4) void k_attn_part4(const int4 *__restrict__ items, const float *__restrict__ qkv, int ldqkv,
+                                                       int nh, int nkv, float scale, const int *__restrict__ pos,
+                                                       uint16_t *const *__restrict__ kc, uint16_t *const *__restrict__ vc,
+                                                       float *__restrict__ part, int pstride) {
+    __shared__ __align__(16) float qs[4 * 128];
+    __shared__ __align__(16) float es[4 * ATM4_EP];
+    __shared__ float red[4][4];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), i16 = lane & 15, quad = lane >> 4;
+    const int4 it = items[blockIdx.x];
+    const int r0 = it.x, g = it.z, kb = it.w, nq = nh / nkv;
+    int n = pos[r0] + 1 - kb * ATT_P;
+    n = n < ATT_P ? n : ATT_P;
+    // the query vectors' load before the cache's (loads complete in order; past nq and past HD: 0)
+    const int qv = (t >> 5) & 3, qd = 4 * (t & 31);
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)(qkv + (size_t)r0 * ldqkv), (short)0, ldqkv * 4, GW_RSRC_DW3);
+    const float4 qx = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+        rq, qv < nq && qd < HD ? ((g * nq + qv) * HD + qd) * 4 : ldqkv * 4, 0, 0));
+    __builtin_amdgcn_sched_barrier(0);
+    const uint16_t *K = kc[r0] + ((size_t)kb * nkv + g) * ATT_P * HD, *V = vc[r0] + ((size_t)kb * nkv + g) * ATT_P * HD;
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)K, (short)0, ((n + ATT_T - 1) & ~(ATT_T - 1)) * HD * 2, GW_RSRC_DW3);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)V, (short)0, n * HD * 2, GW_RSRC_DW3);
+    const int ko = (4 * w + (i16 >> 2)) * 32 * HD + atm_koff<KB>(i16, quad);
+    Attn4K<HD, KB, ATM4_NT> kr;
+    kr.first(rk, ko);
+    const int role = ((int)(blockIdx.x >> 3) + w) & 3; // (0, 2: the folding waves; which ones changes with the block)
+    const int vo = role & 1 ? ATT_P * HD * 2 : attn4_vo<HD>();
+    Attn4V<HD, ATM4_NT> va, vb;
+    va.load(rv, vo, 0);
+    if (t < 128) *(float4 *)(qs + qv * 128 + qd) = qx;
+    __syncthreads();
+    const int p0 = 64 * w + 16 * (i16 >> 2) + 4 * quad;
+    float sc[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+    if (64 * w < n) attn4_scores<HD, KB>(kr, rk, ko, qs, scale, sc, [](int, uint32_t (&)[4][2]) {});
+    const float m = attn4_softmax(sc, w, p0, n, red, es);
+    // (vector vv's part of block kb: HD values o, then m, l)
+    float *const dst = part + ((size_t)r0 * nh + g * nq) * pstride + (size_t)kb * (HD + 2);
+    auto chains = [&](auto half) __attribute__((always_inline)) {
+        const atm_f4 o = attn4_chains<HD, KB, decltype(half)::value>(va, vb, rv, vo, es, n);
+        const int i = lane;
+        if (i < HD / 2) {
+            #pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (r < nq) dst[(size_t)r * pstride + attn4_dim<KB>(i, decltype(half)::value)] = o[r];
+        }
+    };
+    if (role == 0) chains(std::integral_constant<int, 0>{});
+    else if (role == 2) chains(std::integral_constant<int, 1>{});
+    else if (role == 1) {
+        const float l = attn4_l(es), mv = __shfl(m, quad); // (lane i < 4 holds vector i's m)
+        if (i16 == 0 && quad < nq) {
+            float *ml = dst + (size_t)quad * pstride + HD;
+            ml[0] = mv;
+            ml[1] = l;
+        }
+    }
 }
 
 // The attention of the one-row (decode) pass, one block of 1024 threads per (query vector v, kv head g, key block kb),
@@ -1159,6 +1296,131 @@ __global__ __launch_bounds__(ATD_T) void k_attn_decode(const float *__restrict__
         }
         for (; q < n; q++) o = __builtin_fmaf(S[q], KB ? bf2f(vcol[(size_t)q * HD]) : h2f(vcol[(size_t)q * HD]), o);
         part[(size_t)h * pstride + (size_t)kb * (HD + 2) + t] = o;
+    }
+}
+
+// k_attn_decode for long rows (gw_k_attn_decode's choice), one block per (up to 4 of the kv_mul query vectors of kv head g,
+// key block kb): K / V read once per 4 vectors, with k_attn_part4's chains; QK-norm, RoPE and the K / V store as there.
+// The waves normalize and rotate the vectors, one each; a fifth wave makes the row's key and value of head g in the
+// blocks of the last key block and stores them. There the key goes into the operand of the one wave that holds position
+// pos, and the value is the last fma of the o chains (V is read up to pos - 1). Blocks b: g = b % nkv (8 kv heads: one
+// per XCD), then the vectors' group, then kb. 32,702 positions (134 MB): k_attn_decode 124 us, 34.4 here (3.9 TB/s)
+template <int HD, bool KB>
+__global__ __launch_bounds__(320, KB ? 3 : 4) void k_attn_decode4(const float *__restrict__ qkv, int nh, int nkv, float scale,
+                                                       const float *__restrict__ qn, const float *__restrict__ kn,
+                                                       const float *__restrict__ rope, int pos, uint16_t *__restrict__ kl,
+                                                       uint16_t *__restrict__ vl, float *__restrict__ part, int pstride) {
+    constexpr int half = HD / 2;
+    __shared__ __align__(16) float qs[4 * 128];
+    __shared__ __align__(16) float es[4 * ATM4_EP];
+    __shared__ __align__(16) float wx[5][HD];
+    __shared__ float red[4][4];
+    __shared__ uint16_t kx[128], vx[HD];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), i16 = lane & 15, quad = lane >> 4;
+    const int kv_mul = nh / nkv, g = blockIdx.x % nkv, ng = (kv_mul + 3) >> 2, y = blockIdx.x / nkv, v0 = 4 * (y % ng), kb = y / ng;
+    const int nq = kv_mul - v0 < 4 ? kv_mul - v0 : 4, pp = pos % ATT_P;
+    const bool last = kb == pos / ATT_P;
+    const int n = last ? pp + 1 : ATT_P; // positions of this block up to pos
+    // 1. the raw vector of this wave (wave 4: the key; waves past the vectors make vector v0 again, never used), a lane
+    // i < HD / 2 values i and i + HD / 2, and the norm's weights and the rotation: before the cache's loads, which complete
+    // in order behind them
+    const int li = lane < half ? lane : half - 1;
+    const float *cs = rope + (size_t)pos * HD, *xp = qkv + (size_t)(w == 4 ? nh + g : g * kv_mul + v0 + (w < nq ? w : 0)) * HD, *np = w == 4 ? kn : qn;
+    const float xa = xp[li], xb = xp[li + half], na = np[li], nb = np[li + half], rc = cs[li], rs = cs[li + half];
+    const float *vp = qkv + (size_t)(nh + nkv + g) * HD;
+    const float vra = vp[li], vrb = vp[li + half];
+    __builtin_amdgcn_sched_barrier(0);
+    // 2. the cache's K and V
+    const uint16_t *K = kl + ((size_t)kb * nkv + g) * ATT_P * HD, *V = vl + ((size_t)kb * nkv + g) * ATT_P * HD;
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)K, (short)0, ((n + ATT_T - 1) & ~(ATT_T - 1)) * HD * 2, GW_RSRC_DW3);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)V, (short)0, (last ? pp : ATT_P) * HD * 2, GW_RSRC_DW3);
+    const int ko = w < 4 ? (4 * w + (i16 >> 2)) * 32 * HD + atm_koff<KB>(i16, quad) : ATT_P * HD * 2;
+    Attn4K<HD, KB, 0> kr;
+    kr.first(rk, ko);
+    const int vo = w < 2 ? attn4_vo<HD>() : ATT_P * HD * 2; // (waves 0 and 1 fold)
+    Attn4V<HD, 0> va, vb;
+    va.load(rv, vo, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    // 3. QK-norm + RoPE (k_qknorm_rope_store's arithmetic)
+    {
+        float *const wb = wx[w];
+        if (lane < half) wb[lane] = xa, wb[lane + half] = xb;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        float ss = 0.0f, c[HD / 16]; // (chain j: x[j], x[j + 16], ..., then the tree +8 +4 +2 +1: rms_scale_lds)
+        #pragma unroll
+        for (int k = 0; k < HD / 16; k++) c[k] = wb[i16 + 16 * k];
+        #pragma unroll
+        for (int k = 0; k < HD / 16; k++) ss = __builtin_fmaf(c[k], c[k], ss);
+        ss = ss + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ss), 0x108, 0xF, 0xF, true));
+        ss = ss + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ss), 0x104, 0xF, 0xF, true));
+        ss = ss + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ss), 0x102, 0xF, 0xF, true));
+        ss = ss + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ss), 0x101, 0xF, 0xF, true));
+        const float tt = __builtin_fmaf(ss, 1.0f / (float)HD, 1e-6f);
+        const float r = rsqrt_ref(__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(tt))));
+        const float x = (na * xa) * r, z = (nb * xb) * r;
+        const float ys = z * rs, yc = z * rc;
+        const float a = __builtin_fmaf(x, rc, -ys), d = __builtin_fmaf(x, rs, yc);
+        if (w < 4) { // (past nq and past HD: zeros)
+            if (HD < 128 || w >= nq) qs[w * 128 + lane] = qs[w * 128 + 64 + lane] = 0.0f;
+            if (lane < half && w < nq) qs[w * 128 + lane] = a, qs[w * 128 + lane + half] = d;
+        } else if (last && lane < half) {
+            const uint16_t ha = KB ? f2bf_ref(a) : f2h_ref(a), hd = KB ? f2bf_ref(d) : f2h_ref(d);
+            const uint16_t va_ = KB ? f2bf_ref(vra) : f2h_ref(vra), vb_ = KB ? f2bf_ref(vrb) : f2h_ref(vrb);
+            kx[lane] = ha, kx[lane + half] = hd;
+            vx[lane] = va_, vx[lane + half] = vb_;
+            if (v0 == 0) {
+                uint16_t *kd = kl + (((size_t)kb * nkv + g) * ATT_P + (size_t)(pp & ~(ATT_T - 1))) * HD;
+                uint16_t *vd = vl + (((size_t)kb * nkv + g) * ATT_P + pp) * HD;
+                kd[kv_k_at(KB, lane, pp % ATT_T)] = ha, kd[kv_k_at(KB, lane + half, pp % ATT_T)] = hd;
+                vd[kv_v_col(KB, lane)] = va_, vd[kv_v_col(KB, lane + half)] = vb_;
+            }
+        }
+    }
+    __syncthreads();
+    // 4. scores and softmax
+    const int p0 = 64 * w + 16 * (i16 >> 2) + 4 * quad;
+    float sc[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+    if (64 * w < n && w < 4) {
+        const bool own = last && w == pp >> 6, mine = i16 == (pp & 63) >> 2; // (the row's own key: word pp / 2 % 2, half pp % 2)
+        attn4_scores<HD, KB>(kr, rk, ko, qs, scale, sc, [&](int k, uint32_t (&x)[4][2]) {
+            if (!own) return; // (uniform)
+            #pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t h = kx[(32 * quad + 4 * k + j) & (HD - 1)];
+                #pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const uint32_t z = pp & 1 ? (x[j][u] & 0xffffu) | h << 16 : (x[j][u] & 0xffff0000u) | h;
+                    x[j][u] = mine && (pp >> 1 & 1) == u ? z : x[j][u];
+                }
+            }
+        });
+    }
+    const float m = attn4_softmax(sc, w, p0, n, red, es);
+    // 5. o and l
+    float *const dst = part + (size_t)(g * kv_mul + v0) * pstride + (size_t)kb * (HD + 2);
+    auto chains = [&](auto hi) __attribute__((always_inline)) {
+        constexpr int HI = decltype(hi)::value;
+        const atm_f4 o = attn4_chains<HD, KB, HI>(va, vb, rv, vo, es, n);
+        const int i = lane;
+        if (i < HD / 2) {
+            const int d = attn4_dim<KB>(i, HI);
+            const float vn = last ? atm_val<KB>(vx[d], 0) : 0.0f;
+            #pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (r < nq) dst[(size_t)r * pstride + d] = last ? __builtin_fmaf(es[r * ATM4_EP + pp], vn, o[r]) : o[r];
+        }
+    };
+    if (w == 0) chains(std::integral_constant<int, 0>{});
+    else if (w == 1) chains(std::integral_constant<int, 1>{});
+    else if (w == 2) {
+        const float l = attn4_l(es), mv = __shfl(m, quad); // (lane i < 4 holds vector i's m)
+        if (i16 == 0 && quad < nq) {
+            float *ml = dst + (size_t)quad * pstride + HD;
+            ml[0] = mv;
+            ml[1] = l;
+        }
     }
 }
 
@@ -1622,29 +1884,37 @@ int gw_k_unrot_quant(const float *att, int n, int nh, int hd, const int *kvt, in
     return (int)hipGetLastError();
 }
 
-int gw_k_attn_part(const void *items, int nitems, int nq_max, const float *qkv, int ldqkv, int nh, int nkv, int hd, float scale,
-                   const int *pos, uint16_t *const *kc, uint16_t *const *vc, float *part, int pstride, int kbf, hipStream_t s) {
-    int nq = nq_max;
+int gw_k_attn_part(const void *items, int nitems, const float *qkv, int ldqkv, int nh, int nkv, int hd, float scale,
+                   const int *pos, uint16_t *const *kc, uint16_t *const *vc, float *part, int pstride, int kbf, int narrow, hipStream_t s) {
+    // narrow: every item is one row with at most 4 query vectors (k_attn_part4)
+    if (nh % nkv || nh / nkv > (narrow ? 4 : 16)) return (int)hipErrorInvalidValue; // (an item's vectors: one MFMA's columns)
     const int4 *it = (const int4 *)items;
-#define ATT_LAUNCH(Q)                                                                                                   \
-    do {                                                                                                                \
-        if (kbf) GW_LAUNCH((k_attn_part<Q, true>), dim3(nitems), dim3(ATT_TH), 0, s, it, qkv, ldqkv, nh, nkv, hd, scale, pos, kc, vc, part, pstride); \
-        else GW_LAUNCH((k_attn_part<Q, false>), dim3(nitems), dim3(ATT_TH), 0, s, it, qkv, ldqkv, nh, nkv, hd, scale, pos, kc, vc, part, pstride); \
-    } while (0)
-    if (nq <= 1) ATT_LAUNCH(1);
-    else if (nq <= 2) ATT_LAUNCH(2);
-    else if (nq <= 4) ATT_LAUNCH(4);
-    else if (nq <= 8) ATT_LAUNCH(8);
-    else ATT_LAUNCH(16);
-#undef ATT_LAUNCH
+#define ATT_L(KN) GW_LAUNCH((KN), dim3(nitems), dim3(256), 0, s, it, qkv, ldqkv, nh, nkv, scale, pos, kc, vc, part, pstride)
+#define ATT_H(H)                                                                                                        \
+    if (narrow) { if (kbf) ATT_L((k_attn_part4<H, true>)); else ATT_L((k_attn_part4<H, false>)); }                      \
+    else if (kbf) ATT_L((k_attn_part<H, true>)); else ATT_L((k_attn_part<H, false>));
+    if (hd == 128) { ATT_H(128) }
+    else if (hd == 64) { ATT_H(64) }
+    else if (hd == 32) { ATT_H(32) }
+    else return (int)hipErrorInvalidValue;
+#undef ATT_H
+#undef ATT_L
     return (int)hipGetLastError();
 }
 
 int gw_k_attn_decode(const float *qkv, int nh, int nkv, int hd, float scale, const float *qn, const float *kn, const float *rope,
                      int pos, uint16_t *kl, uint16_t *vl, float *part, int pstride, int kbf, hipStream_t s) {
-    int kvm = nh / nkv, nitems = nkv * (pos / ATT_P + 1);
-    dim3 grid(8 * kvm * ((nitems + 7) / 8));
-#define ATD_L(H, B) GW_LAUNCH((k_attn_decode<H, B>), grid, dim3(ATD_T), 0, s, qkv, nh, nkv, scale, qn, kn, rope, pos, kl, vl, part, pstride)
+    // k_attn_decode while its blocks (nh per key block) are at most one per CU, then k_attn_decode4: us per launch
+    // (k_attn_decode / k_attn_decode4), 32 heads: 600 positions 8.6 / 9.8, 2,040 9.8 / 10.5, 2,300 16.5 / 10.6, 8,000 30.9 /
+    // 11.3, 32,702 124 / 34.4; 16 heads: 600 9.1 / 10.1, 4,050 11.1 / 12.6, 5,000 18.0 / 13.4
+    int kvm = nh / nkv, nb = pos / ATT_P + 1, nitems = nkv * nb;
+    const bool wide = nh * nb > gw_device_cus();
+    const dim3 grid(wide ? nkv * ((kvm + 3) / 4) * nb : 8 * kvm * ((nitems + 7) / 8));
+#define ATD_L(H, B)                                                                                                     \
+    do {                                                                                                                \
+        if (wide) GW_LAUNCH((k_attn_decode4<H, B>), grid, dim3(320), 0, s, qkv, nh, nkv, scale, qn, kn, rope, pos, kl, vl, part, pstride); \
+        else GW_LAUNCH((k_attn_decode<H, B>), grid, dim3(ATD_T), 0, s, qkv, nh, nkv, scale, qn, kn, rope, pos, kl, vl, part, pstride); \
+    } while (0)
     if (hd == 128) { if (kbf) ATD_L(128, true); else ATD_L(128, false); }
     else if (hd == 64) { if (kbf) ATD_L(64, true); else ATD_L(64, false); }
     else if (hd == 32) { if (kbf) ATD_L(32, true); else ATD_L(32, false); }

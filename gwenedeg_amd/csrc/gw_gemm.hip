@@ -1112,6 +1112,291 @@ __global__ __launch_bounds__(SK_T * SB, SB == 1 ? 2 : 1) void k_gemm_kq32(SkMats
     }
 }
 
+// Q4_K GEMM of many tiles (prefill): k_gemm_q8l's 64 x 128 blocks (8 waves of 32 x 32, the XCD-aware order) and its copies
+// into LDS by the buffer unit, a stage per super-block (8 groups): the X rows' 256 codes and 8 scales, and the W rows'
+// super-blocks as they are in memory, unpacked by each wave as it reads its MFMA operand (16 bytes of nibbles are the
+// operands of two groups). Two stages in LDS: one is copied while the other is computed. Per group and tile I = the exact sum
+// q x (int8 MFMA), and one outer-product MFMA (v_mfma_f32_32x32x1_f32, two blocks; each result one fp32 product rounded
+// once, as the VALU's multiply) gives xs f0 (f0 = d sc_j) and xf f1 (f1 = dmin m_j, xf = xs (float) sum x, the pairs (xs,
+// xf) made once per stage by the block's threads): term = (xs f0) (float) I - xf f1 (kquants.h:86-109), val = val + term
+// in group order. The VALU bounds it (the fp32 MFMA issues through its pipe too): 4 instructions per output and group and
+// one in two for the products, 370 of them per 32 x 32 tile and group with the unpacking; at 4 waves per SIMD they issue
+// 83 % of the cycles. k_gemm_kq (unpacks into LDS between two barriers per half super-block, 8 instructions per output and
+// group) -> here, us per launch at 512 rows: 19,456 x 2,560 165 -> 142, 9,728 x 2,560 110 -> 86, 4,096 x 2,560 53 -> 37
+// LDS: chunk c of X row r at c ^ (r % 16) of the row's 16; W rows 144 bytes apart (the 16 rows of a read on distinct banks)
+#define KL_PPR(T) ((T) == GW_Q4_K ? 9 : (T) == GW_Q5_K ? 11 : 14) // 16-byte pieces of a super-block
+__global__ __launch_bounds__(512, 4) void k_gemm_kql(SkMats mats, int bstride, int K, const int8_t *__restrict__ X,
+                                                     const float *__restrict__ XS, int ldx, int M, float *out, int ldo,
+                                                     int mode, int MT) {
+    constexpr int TN = 128, NC = TN / 32, NW = 2 * NC, PPR = KL_PPR(GW_Q4_K), PX = 16, PW = PPR * TN / 64, PT = PX + PW + 2, PPW = (PT + NW - 1) / NW;
+    constexpr int OW = 16384, OXS = OW + PW * 1024, STG = OXS + 2048, XXR = 72; // (XXR: bytes per row of (xs, xf) pairs)
+    __shared__ __align__(16) uint8_t sl[2 * STG];
+    __shared__ __align__(16) uint8_t xx[64 * XXR];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), hi = lane >> 5, r32 = lane & 31;
+    const int mi = blockIdx.x >= mats.nb1, b = blockIdx.x - (mi ? mats.nb1 : 0), j = b >> 3, N = mats.N[mi];
+    const int n0 = ((j / MT) * 8 + (b & 7)) * TN, m0 = (j % MT) * 64, S = K >> 8, gx = ldx >> 5;
+    if (n0 >= N) return; // (the grid's padding to 8 column tiles per XCD)
+    const int rowb = S * bstride;
+    const int mr = M - m0 < 64 ? M - m0 : 64, nr = N - n0 < TN ? N - n0 : TN;
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(X + (size_t)m0 * ldx), (short)0, mr * ldx, GW_RSRC_DW3);
+    const __amdgpu_buffer_rsrc_t rxs = __builtin_amdgcn_make_buffer_rsrc((void *)(XS + (size_t)m0 * gx), (short)0, mr * gx * 4, GW_RSRC_DW3);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)(mats.W[mi] + (size_t)n0 * rowb), (short)0, nr * rowb, GW_RSRC_DW3);
+    // this wave's pieces of 1 KB per stage (piece p by wave p % NW; every offset in the per-lane operand, whose range check
+    // makes rows past M / N read 0)
+    int plo[PPW], pvo[PPW], pk[PPW];
+    #pragma unroll
+    for (int i = 0; i < PPW; i++) {
+        const int p = wave + NW * i;
+        if (p < PX) {
+            const int row = 4 * p + (lane >> 4);
+            plo[i] = 1024 * p, pvo[i] = row * ldx + 16 * ((lane & 15) ^ (row & 15)), pk[i] = 0;
+        } else if (p < PX + PW) {
+            const int o = 64 * (p - PX) + lane, row = o / PPR, pc = o % PPR;
+            plo[i] = OW + 1024 * (p - PX), pvo[i] = row * rowb + 16 * pc, pk[i] = 1;
+        } else {
+            const int row = 32 * (p - PX - PW) + (lane >> 1);
+            plo[i] = OXS + 1024 * (p - PX - PW), pvo[i] = (row * gx + 4 * (lane & 1)) * 4, pk[i] = 2;
+        }
+    }
+    auto issue = [&](int st) __attribute__((always_inline)) {
+        uint8_t *bs = sl + (st & 1) * STG;
+        #pragma unroll
+        for (int i = 0; i < PPW; i++)
+            if (wave + NW * i < PT) {
+                if (pk[i] == 0) lq_copy(rx, bs + plo[i], pvo[i] + 256 * st, 16);
+                else if (pk[i] == 1) lq_copy(rw, bs + plo[i], pvo[i] + bstride * st, 16);
+                else lq_copy(rxs, bs + plo[i], pvo[i] + 32 * st, 16);
+            }
+    };
+    const int wm = (wave / NC) * 32, wn = (wave % NC) * 32;
+    float acc[16];
+    #pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+    const int xr = wm + r32, xo = xr * 256, xw = xr & 15, wo = OW + (wn + r32) * (16 * PPR), xso = OXS + xr * 32;
+    const i32x16 z = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+    const f32x32 zf = {};
+    issue(0);
+    for (int st = 0; st < S; st++) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); // (stage st landed, every wave's; stage st - 1 read)
+        if (st + 1 < S) issue(st + 1);
+        const uint8_t *bs = sl + (st & 1) * STG;
+        #pragma unroll
+        for (int o = t; o < 512; o += NW * 64) { // (xs, xs (float) sum x) of row o / 8, group o % 8
+            const int row = o >> 3, g = o & 7;
+            const i32x4 a = *(const i32x4 *)(bs + row * 256 + 16 * ((2 * g) ^ (row & 15))), c = *(const i32x4 *)(bs + row * 256 + 16 * ((2 * g + 1) ^ (row & 15)));
+            int sx = 0;
+            #pragma unroll
+            for (int e = 0; e < 4; e++) sx = __builtin_amdgcn_sdot4(a[e], 0x01010101, sx, false);
+            #pragma unroll
+            for (int e = 0; e < 4; e++) sx = __builtin_amdgcn_sdot4(c[e], 0x01010101, sx, false);
+            const float xs = *(const float *)(bs + OXS + row * 32 + 4 * g);
+            *(float2 *)(xx + row * XXR + 8 * g) = make_float2(xs, xs * (float)sx);
+        }
+        // the 8 sub-blocks' 6-bit values of this lane's half (hi 0: sc_j, 1: m_j) as bytes, and d or dmin
+        const uint4 hd = *(const uint4 *)(bs + wo);
+        const uint32_t a = hi ? hd.z : hd.y, c = hi ? hd.w >> 4 : hd.w;
+        const uint32_t b6[2] = { a & 0x3F3F3F3Fu, (c & 0x0F0F0F0Fu) | ((a >> 2) & 0x30303030u) };
+        const float db = h2f_g((uint16_t)(hi ? hd.x >> 16 : hd.x & 0xffffu));
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); // (the pairs written)
+        #pragma unroll
+        for (int i = 0; i < 4; i++) { // (groups 2 i, 2 i + 1: the low and the high nibbles of 32 bytes)
+            const uint4 q = *(const uint4 *)(bs + wo + 16 + 32 * i + 16 * hi);
+            const uint32_t q4[4] = { q.x, q.y, q.z, q.w };
+            #pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int g = 2 * i + u;
+                const i32x4 A = *(const i32x4 *)(bs + xo + 16 * ((2 * g + hi) ^ xw));
+                i32x4 B;
+                #pragma unroll
+                for (int e = 0; e < 4; e++) B[e] = (int)((u ? q4[e] >> 4 : q4[e]) & 0x0F0F0F0Fu);
+                const i32x16 I = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, B, z, 0, 0, 0);
+                const float ca = *(const float *)(xx + xr * XXR + 8 * g + 4 * hi);
+                const float cb = db * (float)((b6[g >> 2] >> (8 * (g & 3))) & 0xffu);
+                const f32x32 C = __builtin_amdgcn_mfma_f32_32x32x1f32(ca, cb, zf, 0, 0, 0);
+                #pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const float pa = C[r] * (float)I[r];
+                    acc[r] = acc[r] + (pa - C[16 + r]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    out += mats.col[mi];
+    const int n = n0 + wn + r32;
+    #pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int m = m0 + wm + 8 * (r >> 2) + 4 * hi + (r & 3);
+        if (m < M && n < N) {
+            float *o = out + (size_t)m * ldo + n;
+            *o = mode == 1 ? *o + acc[r] : acc[r];
+        }
+    }
+}
+
+// k_gemm_kql's stages and terms for Q4_K, Q5_K and Q6_K in blocks of 32 x 32 outputs, 4 waves of 16 x 16
+// (v_mfma_i32_16x16x32_i8, one group per instruction): a narrow matrix still gives each CU several blocks (4 - 5 fit), and
+// the last round of blocks is short (w2 of a 512-row prompt: 320 blocks of 64 x 64 left three quarters of the CUs with
+// one, 1280 of 32 x 32 are five each). Q4_K, Q5_K: a v_mfma_f32_16x16x1_f32 of 4 blocks gives two groups' products. Q6_K
+// (kquants.h:410-554): per half-group of 16 sum q x - 32 sum x (an MFMA with B = -32 makes the accumulator of the one with
+// the codes q 0 .. 63, so no code is sign-extended); T over the group and T_0 over its first half (B masked), I = sc_0 T_0 +
+// sc_1 (T - T_0) = (sc_0 - sc_1) T_0 + sc_1 T, exact; one 4-block MFMA for 4 groups' xs d. Bound by the VALU as
+// k_gemm_kql (104 cycles per 16 x 16 tile and group, Q6_K 140), at 70 %. us per launch, what ran before -> here:
+//   512 rows: Q6_K 2,560 x 9,728 201 -> 139, 1,024 x 2,560 41 -> 19; Q4_K 2,560 x 4,096 77 -> 42, 5,120 x 2,560 67 -> 51
+//   100 rows: Q6_K 2,560 x 9,728 145 -> 60; Q4_K 4,096 x 2,560 42 -> 16; 40 rows: 44 -> 18 (2,560 x 4,096), 38 -> 12 (1,024)
+//   32 rows: Q6_K 151,936 x 2,560 204 -> 133; Q4_K 19,456 x 2,560 25.7 -> 21.8; 8 rows: 194 -> 125, 28.1 -> 19.4
+template <int TYPE>
+__global__ __launch_bounds__(256, TYPE == GW_Q5_K ? 4 : 5) void k_gemm_kqt(SkMats mats, int bstride, int K, const int8_t *__restrict__ X,
+                                                     const float *__restrict__ XS, int ldx, int M, float *out, int ldo,
+                                                     int mode, int MT) {
+    constexpr int PPR = KL_PPR(TYPE), PX = 8, PW = (PPR * 32 + 63) / 64, PT = PX + PW + 1, PPW = (PT + 3) / 4;
+    constexpr int OW = 8192, OXS = OW + PW * 1024, STG = OXS + 1024, XXR = 80; // (XXR: bytes per row of (xs, xf) pairs)
+    constexpr int PB = (TYPE == GW_Q4_K ? GW_Q4K_BYTES : TYPE == GW_Q5_K ? GW_Q5K_BYTES : GW_Q6K_DEV) / 16;
+    __shared__ __align__(16) uint8_t sl[2 * STG + (TYPE == GW_Q6_K ? 0 : 32 * XXR)];
+    uint8_t *const xx = sl + 2 * STG;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l16 = lane & 15, q4 = lane >> 4;
+    const int mi = blockIdx.x >= mats.nb1, b = blockIdx.x - (mi ? mats.nb1 : 0), j = b >> 3, N = mats.N[mi];
+    const int n0 = ((j / MT) * 8 + (b & 7)) * 32, m0 = (j % MT) * 32, S = K >> 8, gx = ldx >> 5;
+    if (n0 >= N) return; // (the grid's padding to 8 column tiles per XCD)
+    const int rowb = S * bstride;
+    const int mr = M - m0 < 32 ? M - m0 : 32, nr = N - n0 < 32 ? N - n0 : 32;
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(X + (size_t)m0 * ldx), (short)0, mr * ldx, GW_RSRC_DW3);
+    const __amdgpu_buffer_rsrc_t rxs = __builtin_amdgcn_make_buffer_rsrc((void *)(XS + (size_t)m0 * gx), (short)0, mr * gx * 4, GW_RSRC_DW3);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)(mats.W[mi] + (size_t)n0 * rowb), (short)0, nr * rowb, GW_RSRC_DW3);
+    int plo[PPW], pvo[PPW], pk[PPW];
+    #pragma unroll
+    for (int i = 0; i < PPW; i++) {
+        const int p = wave + 4 * i;
+        if (p < PX) {
+            const int row = 4 * p + (lane >> 4);
+            plo[i] = 1024 * p, pvo[i] = row * ldx + 16 * ((lane & 15) ^ (row & 15)), pk[i] = 0;
+        } else if (p < PX + PW) {
+            const int o = 64 * (p - PX) + lane, row = o / PPR, pc = o % PPR; // (rows 32 ..: past the tile, not copied)
+            plo[i] = OW + 1024 * (p - PX), pvo[i] = pc < PB && row < 32 ? row * rowb + 16 * pc : 0x7f000000, pk[i] = 1;
+        } else {
+            plo[i] = OXS, pvo[i] = ((lane >> 1) * gx + 4 * (lane & 1)) * 4, pk[i] = 2;
+        }
+    }
+    auto issue = [&](int st) __attribute__((always_inline)) {
+        uint8_t *bs = sl + (st & 1) * STG;
+        #pragma unroll
+        for (int i = 0; i < PPW; i++)
+            if (wave + 4 * i < PT) {
+                if (pk[i] == 0) lq_copy(rx, bs + plo[i], pvo[i] + 256 * st, 16);
+                else if (pk[i] == 1) lq_copy(rw, bs + plo[i], pvo[i] + bstride * st, 16);
+                else lq_copy(rxs, bs + plo[i], pvo[i] + 32 * st, 16);
+            }
+    };
+    const int wm = (wave >> 1) * 16, wn = (wave & 1) * 16;
+    float acc[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+    const int xr = wm + l16, xo = xr * 256 + 8 * (q4 & 1), xw = xr & 15, wo = OW + (wn + l16) * (16 * PPR);
+    const i32x4 z = { 0, 0, 0, 0 };
+    const f32x16 zf = {};
+    issue(0);
+    for (int st = 0; st < S; st++) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); // (stage st landed, every wave's; stage st - 1 read)
+        if (st + 1 < S) issue(st + 1);
+        const uint8_t *bs = sl + (st & 1) * STG;
+        if constexpr (TYPE != GW_Q6_K) {
+            { // (xs, xs (float) sum x) of row t / 8, group t % 8
+                const int row = t >> 3, g = t & 7;
+                const i32x4 a = *(const i32x4 *)(bs + row * 256 + 16 * ((2 * g) ^ (row & 15))), c = *(const i32x4 *)(bs + row * 256 + 16 * ((2 * g + 1) ^ (row & 15)));
+                int sx = 0;
+                #pragma unroll
+                for (int e = 0; e < 4; e++) sx = __builtin_amdgcn_sdot4(a[e], 0x01010101, sx, false);
+                #pragma unroll
+                for (int e = 0; e < 4; e++) sx = __builtin_amdgcn_sdot4(c[e], 0x01010101, sx, false);
+                const float xs = *(const float *)(bs + OXS + row * 32 + 4 * g);
+                *(float2 *)(xx + row * XXR + 8 * g) = make_float2(xs, xs * (float)sx);
+            }
+            // lane quad q4: group 2 i + q4 / 2, q4 % 2 the product xs f0 or xf f1: its 6-bit values and d or dmin
+            const uint4 hd = *(const uint4 *)(bs + wo);
+            const uint32_t a = q4 & 1 ? hd.z : hd.y, c = q4 & 1 ? hd.w >> 4 : hd.w;
+            const int sh = 8 * (q4 >> 1);
+            const uint32_t b6[2] = { (a & 0x3F3F3F3Fu) >> sh, ((c & 0x0F0F0F0Fu) | ((a >> 2) & 0x30303030u)) >> sh };
+            const float db = h2f_g((uint16_t)(q4 & 1 ? hd.x >> 16 : hd.x & 0xffffu));
+            uint2 qh = make_uint2(0, 0);
+            if constexpr (TYPE == GW_Q5_K) qh = *(const uint2 *)(bs + wo + 16 + 8 * q4);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            #pragma unroll
+            for (int i = 0; i < 4; i++) { // (groups 2 i, 2 i + 1: the low and the high nibbles of 32 bytes)
+                const uint2 q = *(const uint2 *)(bs + wo + (TYPE == GW_Q5_K ? 48 : 16) + 32 * i + 8 * q4);
+                const uint32_t qw[2] = { q.x, q.y }, hw[2] = { qh.x, qh.y };
+                const float ca = *(const float *)(xx + xr * XXR + 16 * i + 4 * q4);
+                const float cb = db * (float)((b6[i >> 1] >> (16 * (i & 1))) & 0xffu);
+                const f32x16 C = __builtin_amdgcn_mfma_f32_16x16x1f32(ca, cb, zf, 0, 0, 0);
+                i32x4 I[2];
+                #pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const int g = 2 * i + u;
+                    uint32_t v[2];
+                    #pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        v[e] = (u ? qw[e] >> 4 : qw[e]) & 0x0F0F0F0Fu;
+                        if constexpr (TYPE == GW_Q5_K) v[e] |= (g < 4 ? hw[e] << (4 - g) : hw[e] >> (g - 4)) & 0x10101010u;
+                    }
+                    const i64 A = *(const i64 *)(bs + xo + 16 * ((2 * g + (q4 >> 1)) ^ xw));
+                    I[u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, (i64)v[0] | (i64)v[1] << 32, z, 0, 0, 0);
+                }
+                #pragma unroll
+                for (int u = 0; u < 2; u++)
+                    #pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float pa = C[8 * u + r] * (float)I[u][r];
+                        acc[r] = acc[r] + (pa - C[8 * u + 4 + r]);
+                    }
+            }
+        } else {
+            const uint4 scv = *(const uint4 *)(bs + wo + 192);
+            const uint32_t sc4[4] = { scv.x, scv.y, scv.z, scv.w };
+            const float d = h2f_g((uint16_t)(*(const uint32_t *)(bs + wo + 208) & 0xffffu));
+            const i64 m32 = (i64)0xE0E0E0E0E0E0E0E0ll, m0h = q4 < 2 ? m32 : 0;
+            const uint32_t hm = q4 < 2 ? 0xffffffffu : 0u;
+            #pragma unroll
+            for (int nn = 0; nn < 2; nn++) {
+                const uint2 h = *(const uint2 *)(bs + wo + 128 + 32 * nn + 8 * q4);
+                const uint2 l0 = *(const uint2 *)(bs + wo + 64 * nn + 8 * q4), l1 = *(const uint2 *)(bs + wo + 64 * nn + 32 + 8 * q4);
+                const uint32_t hw[2] = { h.x, h.y }, lw[2][2] = { { l0.x, l0.y }, { l1.x, l1.y } };
+                const float ca = *(const float *)(bs + OXS + xr * 32 + 16 * nn + 4 * q4);
+                const f32x16 C = __builtin_amdgcn_mfma_f32_16x16x1f32(ca, d, zf, 0, 0, 0);
+                #pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    const int g = 4 * nn + p;
+                    uint32_t q[2];
+                    #pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        const uint32_t hb = p < 2 ? hw[e] << (4 - 2 * p) : hw[e] >> (2 * p - 4);
+                        q[e] = ((p >> 1 ? lw[p & 1][e] >> 4 : lw[p & 1][e]) & 0x0F0F0F0Fu) | (hb & 0x30303030u);
+                    }
+                    const i64 A = *(const i64 *)(bs + xo + 16 * ((2 * g + (q4 >> 1)) ^ xw));
+                    const i64 B = (i64)q[0] | (i64)q[1] << 32, B0 = (i64)(q[0] & hm) | (i64)(q[1] & hm) << 32;
+                    i32x4 T = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, m32, z, 0, 0, 0);
+                    i32x4 T0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, m0h, z, 0, 0, 0);
+                    T = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, B, T, 0, 0, 0);
+                    T0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, B0, T0, 0, 0, 0);
+                    const uint32_t sw = sc4[g >> 1] >> (16 * (g & 1));
+                    const int s1 = (int)(int8_t)((sw >> 8) & 0xffu), sd = (int)(int8_t)(sw & 0xffu) - s1;
+                    #pragma unroll
+                    for (int r = 0; r < 4; r++) { // (|sd| <= 255, |T_0| < 2^17, |T| < 2^18)
+                        const int I = __mul24(sd, T0[r]) + __mul24(s1, T[r]);
+                        acc[r] = acc[r] + C[4 * p + r] * (float)I;
+                    }
+                }
+            }
+        }
+    }
+    out += mats.col[mi];
+    const int n = n0 + wn + l16;
+    #pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int m = m0 + wm + 4 * q4 + r;
+        if (m < M && n < N) {
+            float *o = out + (size_t)m * ldo + n;
+            *o = mode == 1 ? *o + acc[r] : acc[r];
+        }
+    }
+}
+
 // --------------------------------------------------------------------------------------------- K-quants
 
 // The batched GEMV of every weight format: out[m * ldo + row] (+)= W row . X row m for M <= 8 activation rows, R weight
@@ -1932,10 +2217,59 @@ static int launch_kq32(const GwMat *a, const GwMat *b, int col_b, const int8_t *
     return (int)hipGetLastError();
 }
 
+static int kql_takes(const GwMat *w, int rows, const int8_t *xq, const float *xs, int ldx, int M) {
+    // the LDS-copied K-quant GEMMs for w (rows: its rows, or those of the two matrices of a launch): 2 k_gemm_kql, 1
+    // k_gemm_kqt, 0 neither (16-byte copies: aligned rows). Up to 32 rows k_gemm_kqt where its 32 x 32 tiles are more than
+    // one per CU, from 6 rows (us, GEMV / k_gemm_kqt: Q4_K 19,456 x 2,560 at 5 rows 19.0 / 19.4, 6 19.6 / 18.4, 8 28 / 19;
+    // k_gemm_kq32 / k_gemm_kqt at 32 rows: 9,728 x 2,560 (304 tiles) 17.2 / 15.6, 5,120 x 2,560 (160) 11.1 / 13.0), and for
+    // Q5_K, which k_gemm_kq32 does not take, above 8. Above 32 rows: k_gemm_kql (Q4_K) where its 64 x 128 blocks fill at
+    // least 78 % of the CU rounds they take (k_gemm_kql / k_gemm_kqt: 256 blocks 37 / 42, 304 54.9 / 50.9, 320 53.8 / 51.2, 608
+    // 86 / 93, 1,216 142 / 178), else k_gemm_kqt; Q6_K where k_gemm_kq's 64 x 128 tiles are 4 per CU or more stays there
+    // (16,384 x 2,560 at 512 rows 171 / 208; at 256, below that, 100 / 102)
+    if ((w->type != GW_Q4_K && w->type != GW_Q5_K && w->type != GW_Q6_K) || g_tile_rows ||
+        (((uintptr_t)w->blocks | (uintptr_t)xq | (uintptr_t)xs) & 15) || ldx % 128 || (size_t)128 * (w->cols >> 8) * w->bstride >= ((size_t)1 << 30))
+        return 0;
+    const size_t cus = (size_t)gw_device_cus(), nb = (size_t)((rows + 127) / 128) * ((M + 63) / 64);
+    if (M <= 32) {
+        if (w->type == GW_Q5_K) return M > 8 || (M >= 6 && (size_t)(rows + 31) / 32 > cus);
+        return M >= 6 && (size_t)(rows + 31) / 32 > cus && !g_kq16 && !g_kq32_nqr && !g_kq32_sb;
+    }
+    if (w->type == GW_Q6_K) return nb < 4 * cus;
+    return w->type == GW_Q4_K && nb * 100 >= (nb + cus - 1) / cus * cus * 78 ? 2 : 1;
+}
+
+static int launch_kql(int kern, const GwMat *a, const GwMat *b, int col_b, const int8_t *xq, const float *xs, int ldx, int M,
+                      float *out, int ldo, int mode, hipStream_t s) {
+    // a, and b (NULL: none; same type and width as a) written from column col_b of out
+    hipEvent_t e0, e1;
+    gw_take_launch_events(&e0, &e1);
+    const int tn = kern == 2 ? 128 : 32, mt = kern == 2 ? (M + 63) / 64 : (M + 31) / 32;
+    auto nblk = [&](int rows) { return (rows + 8 * tn - 1) / (8 * tn) * 8 * mt; }; // (column tiles padded to 8 per XCD)
+    SkMats m;
+    m.W[0] = a->blocks;
+    m.N[0] = a->rows;
+    m.col[0] = 0;
+    m.nb1 = nblk(a->rows);
+    m.W[1] = b ? b->blocks : a->blocks;
+    m.N[1] = b ? b->rows : a->rows;
+    m.col[1] = b ? col_b : 0;
+    const dim3 grid(m.nb1 + (b ? nblk(b->rows) : 0));
+#define KL_L(KN, T) hipExtLaunchKernelGGL((KN), grid, dim3(T), 0, s, e0, e1, 0, m, a->bstride, a->cols, xq, xs, ldx, M, out, ldo, mode, mt)
+    if (kern == 2) KL_L(k_gemm_kql, 512);
+    else if (a->type == GW_Q4_K) KL_L(k_gemm_kqt<GW_Q4_K>, 256);
+    else if (a->type == GW_Q5_K) KL_L(k_gemm_kqt<GW_Q5_K>, 256);
+    else KL_L(k_gemm_kqt<GW_Q6_K>, 256);
+#undef KL_L
+    return (int)hipGetLastError();
+}
+
 int gw_k_matmul2(const GwMat *a, const GwMat *b, int col_b, const int8_t *xq, const float *xs, int ldx, int M, float *out,
                  int ldo, int mode, hipStream_t s) {
-    /* a and b (b from column col_b of out) in one launch where the 9 .. 32-row K-quant GEMM takes both with one type
-     * and width; else -1 and nothing launched (the caller launches them one by one) */
+    /* a and b (b from column col_b of out) in one launch where one of the K-quant GEMMs (9 .. 32 rows, above 32) takes
+     * both with one type and width; else -1 and nothing launched (the caller launches them one by one) */
+    const bool like = a->type == b->type && a->cols == b->cols && a->bstride == b->bstride && !((uintptr_t)b->blocks & 15);
+    const int kern = like ? kql_takes(a, a->rows + b->rows, xq, xs, ldx, M) : 0;
+    if (kern) return launch_kql(kern, a, b, col_b, xq, xs, ldx, M, out, ldo, mode, s);
     if (kq32_takes(a, M) && kq32_takes(b, M) && a->type == b->type && a->cols == b->cols && a->bstride == b->bstride)
         return launch_kq32(a, b, col_b, xq, xs, ldx, M, out, ldo, mode, s);
     return -1;
@@ -1979,6 +2313,8 @@ int gw_k_matmul(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int 
     }
     if (w->type == GW_Q8_0)
         return launch_gemv_mr<GW_Q8_0>((const uint8_t *)w->codes, w->scales, w->rows, w->cols, 0, xq, xs, ldx, M, out, ldo, mode, s);
+    const int kern = kql_takes(w, w->rows, xq, xs, ldx, M);
+    if (kern) return launch_kql(kern, w, NULL, 0, xq, xs, ldx, M, out, ldo, mode, s);
     if (kq32_takes(w, M)) return launch_kq32(w, NULL, 0, xq, xs, ldx, M, out, ldo, mode, s);
     // K-quants above 32 rows: the MFMA GEMM where it has 64 blocks or more (a block streams its 128 rows' full K in
     // order, so a narrow matrix leaves the device idle) or its row tile is forced, else the batched GEMV in passes of

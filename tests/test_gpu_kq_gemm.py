@@ -1,0 +1,51 @@
+"""The LDS-copied K-quant GEMMs (k_gemm_kql, k_gemm_kqt) against the oracle bit for bit, at the edges of their tiles, stages
+and dispatch."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    import gwenedeg_amd as gw
+    return torch, gw
+
+
+# 12 Q4_K, 13 Q5_K, 14 Q6_K. k_gemm_kqt: above 32 rows, one to several stages (K / 256), row and column remainders of its
+# 32 x 32 tiles; 6 .. 32 rows once its tiles are more than one per CU (8,193 weight rows); Q5_K from 9 rows. k_gemm_kql (Q4_K):
+# 64 x 128 blocks that fill the CUs (25,700 weight rows, 33 rows; 1 row past a block). 131,100-row
+# Q6_K at 33 rows keeps k_gemm_kq (4 blocks per CU)
+@pytest.mark.parametrize("typ,N,K,M", [
+    (12, 31, 256, 33), (12, 33, 512, 64), (12, 200, 2560, 65), (12, 1000, 768, 97),
+    (13, 33, 256, 33), (13, 200, 1024, 9), (13, 70, 512, 32), (13, 129, 768, 70),
+    (14, 1, 256, 33), (14, 33, 512, 40), (14, 200, 2560, 65), (14, 130, 9728, 36),
+    (12, 8193, 256, 6), (12, 8193, 512, 32), (13, 8193, 256, 7), (14, 8193, 256, 6), (14, 8200, 512, 31),
+    (12, 25700, 256, 33), (12, 25601, 512, 65), (12, 12801, 768, 129),
+    (14, 131100, 256, 33)])
+def test_lds_copied_kq_gemm_bitexact(dev, typ, N, K, M):
+    torch, gw = dev
+    from oracle import oracle as orc
+    from gwenedeg_amd import synth
+    rng = np.random.default_rng(typ * 1000 + N + M)
+    sl = synth.synth_library()
+    rb = sl.gw_synth_row_bytes(typ, K)
+    base = np.zeros((min(N, 300), rb), np.uint8)  # (300 distinct rows, repeated shifted by one per repetition)
+    w = rng.normal(0, 0.02, size=(len(base), K)).astype(np.float32)
+    for r in range(len(base)):
+        sl.gw_synth_encode_row(typ, base[r].ctypes.data, w[r].ctypes.data, K)
+    idx = (np.arange(N) + np.arange(N) // len(base)) % len(base)
+    xq, xs = orc.quantize(rng.normal(0, 1, size=(M, K)).astype(np.float32))
+    xq[0, :64] = 127           # the largest group sums
+    xq[M - 1, :32], xs[M - 1, 0] = 0, 0.0
+    ref = orc.kq_matmul(typ, base, xq, xs, len(base), K)[:, idx]
+    buf = torch.from_numpy(base[idx].reshape(-1)).cuda()
+    out = torch.full((M + 1, N), 7.0, dtype=torch.float32, device="cuda")
+    XQ, XS = torch.from_numpy(xq).cuda(), torch.from_numpy(xs).cuda()
+    assert gw.lib.gw_kq_matmul(out.data_ptr(), typ, buf.data_ptr(), N, K, XQ.data_ptr(), XS.data_ptr(), M, None) == 0
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:M].view(np.uint32), ref.view(np.uint32)), f"max diff {np.abs(got[:M] - ref).max()}"
+    assert (got[M] == 7.0).all()

@@ -708,6 +708,18 @@ static int fused_shape(const RqModel *m) {
     return !m->kq && dim <= 4096 && H <= 12288 && q <= 4096 && dim % 64 == 0 && H % 64 == 0 && q % 64 == 0;
 }
 
+static int fusedk_shape(const RqModel *m) {
+    /* a K-quant model whose every matmul the fused single-row K-quant GEMVs take (Q4_K, Q5_K, Q6_K: k_gemvk) */
+    if (!m->kq || !gw_k_gemvk_ok(GW_GK_NORM, &m->cls, 1, 0)) return 0;
+    for (int l = 0; l < m->n_layers; l++) {
+        const GwLayer *y = &m->layer[l];
+        if (y->nqkv != 3 || y->nw13 != 2 || !gw_k_gemvk_ok(GW_GK_NORM, y->qkv, 3, 0) || !gw_k_gemvk_ok(GW_GK_COMBINE, &y->wo, 1, 0) ||
+            !gw_k_gemvk_ok(GW_GK_NORM, y->w13, 2, 1) || !gw_k_gemvk_ok(GW_GK_QF, &y->w2, 1, 0))
+            return 0;
+    }
+    return 1;
+}
+
 typedef struct { int x, y, z, w; } Item; /* attention work item: first row, rows, kv head, key block */
 
 typedef struct {
@@ -739,7 +751,7 @@ static int run_mm(RqCtx *c, const GwMat *w, int nmat, const int8_t *xq, const fl
 #define KCHK(x) do { if (x) return ctx_fail(c, RQ_ERR_STATE, "kernel launch failed: %s", #x); } while (0)
 
 static int fused_layer(RqCtx *c, int l, RqSeq *sq, int pos, const int *pos_d) {
-    /* layer l of the one-row pass of an all-Q8_0 model (the fused decode sequence, x in place): qkv GEMV (rmsnorm +
+    /* layer l of the one-row pass of an all-Q8_0 model, or of a K-quant one (the fused decode sequence, x in place): qkv GEMV (rmsnorm +
      * quantize prologue) -> attention (QK-norm, RoPE, K / V store inside) -> wo GEMV (combine prologue, + residual) ->
      * w1 / w3 GEMV (rmsnorm prologue, SwiGLU epilogue) -> w2 GEMV (+ residual). pos: the row's position (pos_d: the
      * same on the device, for the combine kernel past GW_GV_NBMAX key blocks) */
@@ -750,25 +762,54 @@ static int fused_layer(RqCtx *c, int l, RqSeq *sq, int pos, const int *pos_d) {
     /* (the matmul after w2: the next layer's qkv, or after the last layer the classifier) */
     const GwMat *nx = l + 1 < m->n_layers ? &m->layer[l + 1].qkv[0] : &m->cls;
     const int nxr = l + 1 < m->n_layers ? GW_GV_R_QKV : GW_GV_R_CLS;
+    const int kq = m->kq; /* (a K-quant model, fusedk_shape: k_gemvk, with the same prologues and epilogues) */
+    GwGkIn in = { 0 };
     pf_mark(c, GW_PF_QKV);
-    KCHK(gw_k_gemv1_norm(&y->qkv[0], GW_GV_R_QKV, c->x, y->att_norm, c->qkv, 0, 0, &y->wo, GW_GV_R_WO, s));
+    in.x = c->x, in.nw = y->att_norm;
+    if (kq) KCHK(gw_k_gemvk(GW_GK_NORM, y->qkv, 3, 0, &in, c->qkv, 0, s));
+    else KCHK(gw_k_gemv1_norm(&y->qkv[0], GW_GV_R_QKV, c->x, y->att_norm, c->qkv, 0, 0, &y->wo, GW_GV_R_WO, s));
     pf_mark(c, GW_PF_ATT);
     KCHK(gw_k_attn_decode(c->qkv, nh, m->n_kv_heads, hd, m->att_scale, y->q_norm, y->k_norm, m->rope, pos,
                           seq_layer(sq, l, 0), seq_layer(sq, l, 1), c->part,
                           c->pstride, sq->kvt == RQ_KV_BF16, s));
     if (nb <= GW_GV_NBMAX) {
         pf_mark(c, GW_PF_WO);
-        KCHK(gw_k_gemv1_combine(&y->wo, GW_GV_R_WO, c->part, c->pstride, hd, nb, c->x, 1, &y->w13[0], GW_GV_R_W13, s));
+        in.part = c->part, in.pstride = c->pstride, in.hd = hd, in.nb = nb;
+        if (kq) KCHK(gw_k_gemvk(GW_GK_COMBINE, &y->wo, 1, 0, &in, c->x, 1, s));
+        else KCHK(gw_k_gemv1_combine(&y->wo, GW_GV_R_WO, c->part, c->pstride, hd, nb, c->x, 1, &y->w13[0], GW_GV_R_W13, s));
     } else {
         pf_mark(c, GW_PF_COMBINE);
         KCHK(gw_k_attn_combine_quant(c->part, c->pstride, nh, hd, pos_d, 1, nb, c->xq, c->xs, c->kmax, NULL, s));
         pf_mark(c, GW_PF_WO);
-        KCHK(gw_k_gemv1_q(&y->wo, GW_GV_R_WO, c->xq, c->xs, c->x, 1, &y->w13[0], GW_GV_R_W13, s));
+        in.xq = c->xq, in.xs = c->xs;
+        if (kq) KCHK(gw_k_gemvk(GW_GK_Q, &y->wo, 1, 0, &in, c->x, 1, s));
+        else KCHK(gw_k_gemv1_q(&y->wo, GW_GV_R_WO, c->xq, c->xs, c->x, 1, &y->w13[0], GW_GV_R_W13, s));
     }
     pf_mark(c, GW_PF_W13);
-    KCHK(gw_k_gemv1_norm(&y->w13[0], GW_GV_R_W13, c->x, y->ffn_norm, c->hb, 0, y->w13_il, &y->w2, GW_GV_R_W2, s));
+    in.x = c->x, in.nw = y->ffn_norm;
+    if (kq) KCHK(gw_k_gemvk(GW_GK_NORM, y->w13, 2, 1, &in, c->hb, 0, s));
+    else KCHK(gw_k_gemv1_norm(&y->w13[0], GW_GV_R_W13, c->x, y->ffn_norm, c->hb, 0, y->w13_il, &y->w2, GW_GV_R_W2, s));
     pf_mark(c, GW_PF_W2);
-    KCHK(gw_k_gemv1_qf(&y->w2, GW_GV_R_W2, c->hb, c->x, 1, nx, nxr, s));
+    in.x = c->hb;
+    if (kq) KCHK(gw_k_gemvk(GW_GK_QF, &y->w2, 1, 0, &in, c->x, 1, s));
+    else KCHK(gw_k_gemv1_qf(&y->w2, GW_GV_R_W2, c->hb, c->x, 1, nx, nxr, s));
+    return RQ_OK;
+}
+
+static int fused_cls(RqCtx *c) {
+    /* the classifier of the one-row pass, with the final rmsnorm of x in its prologue */
+    const RqModel *m = c->m;
+    GwGkIn in = { 0 };
+    in.x = c->x, in.nw = m->final_norm;
+    if (m->kq) KCHK(gw_k_gemvk(GW_GK_NORM, &m->cls, 1, 0, &in, c->logits_d, 0, c->stream));
+    else KCHK(gw_k_gemv1_norm(&m->cls, GW_GV_R_CLS, c->x, m->final_norm, c->logits_d, 0, 0, NULL, 0, c->stream));
+    return RQ_OK;
+}
+
+static int embed_rows(RqCtx *c, const int *tok_d, int n) {
+    const RqModel *m = c->m;
+    if (m->embd.type == GW_Q8_0) KCHK(gw_k_embed_q8(c->x, m->dim, (const uint8_t *)m->embd.codes, m->embd.scales, tok_d, n, c->stream));
+    else KCHK(gw_k_embed_kq(c->x, m->dim, m->embd.type, m->embd.blocks, m->embd.bstride, tok_d, n, c->stream));
     return RQ_OK;
 }
 
@@ -858,26 +899,21 @@ static int fw_pass(RqCtx *c, Pass *P, float *out) {
     c->nev = 0;
     c->kt_multi = n > 1;
     pf_mark(c, GW_PF_EMBED);
-    if (m->embd.type == GW_Q8_0) KCHK(gw_k_embed_q8(c->x, dim, (const uint8_t *)m->embd.codes, m->embd.scales, tok_d, n, s));
-    else KCHK(gw_k_embed_kq(c->x, dim, m->embd.type, m->embd.blocks, m->embd.bstride, tok_d, n, s));
-    /* one row of an all-Q8_0 model: the fused decode sequence (gw_gemv.hip: each matmul computes its activation from
-     * the producer's fp32 output; the residual adds go straight into x) */
-    int fused = n == 1 && fused_shape(m) && !nqz, fused_att = fused && (hd == 128 || hd == 64 || hd == 32);
+    if ((rc = embed_rows(c, tok_d, n)) != RQ_OK) return rc;
+    /* one row of an all-Q8_0 model, or of a Q4_K / Q5_K / Q6_K one: the fused decode sequence (gw_gemv.hip: each matmul
+     * computes its activation from the producer's fp32 output; the residual adds go straight into x; head_dim is 32, 64
+     * or 128: rq_model_load) */
+    const int fused = n == 1 && !nqz && (fused_shape(m) || fusedk_shape(m));
     for (int l = 0; l < L; l++) {
         const GwLayer *y = &m->layer[l];
-        if (fused_att) {
+        if (fused) {
             if ((rc = fused_layer(c, l, P->seq[0], P->pos[0], pos_d)) != RQ_OK) return rc;
             continue;
         }
-        if (fused) {
-            pf_mark(c, GW_PF_QKV);
-            KCHK(gw_k_gemv1_norm(&y->qkv[0], GW_GV_R_QKV, c->x, y->att_norm, c->qkv, 0, 0, NULL, 0, s));
-        } else {
-            pf_mark(c, GW_PF_NORM);
-            KCHK(gw_k_rmsnorm_quant(c->x, l ? c->xb : NULL, dim, y->att_norm, NULL, n, c->xq, c->xs, K, NULL, s));
-            pf_mark(c, GW_PF_QKV);
-            if ((rc = run_mm(c, y->qkv, y->nqkv, c->xq, c->xs, K, n, c->qkv, c->ldqkv, 0)) != RQ_OK) return rc;
-        }
+        pf_mark(c, GW_PF_NORM);
+        KCHK(gw_k_rmsnorm_quant(c->x, l ? c->xb : NULL, dim, y->att_norm, NULL, n, c->xq, c->xs, K, NULL, s));
+        pf_mark(c, GW_PF_QKV);
+        if ((rc = run_mm(c, y->qkv, y->nqkv, c->xq, c->xs, K, n, c->qkv, c->ldqkv, 0)) != RQ_OK) return rc;
         pf_mark(c, GW_PF_ROPE);
         KCHK(gw_k_qknorm_rope_store(c->qkv, c->ldqkv, n, nh, nkv, hd, y->q_norm, y->k_norm, m->rope, pos_d,
                                     kc_d + (size_t)l * n, vc_d + (size_t)l * n, nbf || nqz ? kvt_d : NULL, s));
@@ -892,22 +928,6 @@ static int fw_pass(RqCtx *c, Pass *P, float *out) {
                 KCHK(gw_k_attn_part((const Item *)items_d + off, gcnt[grp], c->qkv, c->ldqkv, nh, nkv, hd,
                                     m->att_scale, pos_d, kc_d + (size_t)l * n, vc_d + (size_t)l * n, c->part, c->pstride,
                                     grp >> 1, !(grp & 1), s));
-        }
-        if (fused) {
-            if (nbmax <= GW_GV_NBMAX) {
-                pf_mark(c, GW_PF_WO);
-                KCHK(gw_k_gemv1_combine(&y->wo, GW_GV_R_WO, c->part, c->pstride, hd, nbmax, c->x, 1, NULL, 0, s));
-            } else {
-                pf_mark(c, GW_PF_COMBINE);
-                KCHK(gw_k_attn_combine_quant(c->part, c->pstride, nh, hd, pos_d, n, nbmax, c->xq, c->xs, K, NULL, s));
-                pf_mark(c, GW_PF_WO);
-                KCHK(gw_k_gemv1_q(&y->wo, GW_GV_R_WO, c->xq, c->xs, c->x, 1, NULL, 0, s));
-            }
-            pf_mark(c, GW_PF_W13);
-            KCHK(gw_k_gemv1_norm(&y->w13[0], GW_GV_R_W13, c->x, y->ffn_norm, c->hb, 0, y->w13_il, NULL, 0, s));
-            pf_mark(c, GW_PF_W2);
-            KCHK(gw_k_gemv1_qf(&y->w2, GW_GV_R_W2, c->hb, c->x, 1, NULL, 0, s));
-            continue;
         }
         pf_mark(c, GW_PF_COMBINE);
         /* (rows of quantized caches: the combined o' into the free qkv buffer, then o = D H o' / hd quantized over theirs) */
@@ -933,7 +953,7 @@ static int fw_pass(RqCtx *c, Pass *P, float *out) {
     }
     if (fused && P->nsel == 1 && !P->want_hidden) { /* the final rmsnorm computed by the classifier's GEMV itself */
         pf_mark(c, GW_PF_CLS);
-        KCHK(gw_k_gemv1_norm(&m->cls, GW_GV_R_CLS, c->x, m->final_norm, c->logits_d, 0, 0, NULL, 0, s));
+        if ((rc = fused_cls(c)) != RQ_OK) return rc;
     } else if (P->nsel > 0) {
         pf_mark(c, GW_PF_NORM);
         KCHK(gw_k_rmsnorm_quant(c->x, resid_done ? NULL : c->xb, dim, m->final_norm, sel_d, P->nsel, c->xq, c->xs, K, NULL, s));
@@ -1038,8 +1058,7 @@ int gw_decode_greedy(RqCtx *c, RqSeq *s, int token, int n, int *tokens) {
     if (n < 1 || !tokens) return ctx_fail(c, RQ_ERR_ARG, "bad greedy arguments (n %d)", n);
     if (token < 0 || token >= m->vocab) return ctx_fail(c, RQ_ERR_ARG, "token %d out of range", token);
     if (s->len + n > s->cap) return ctx_fail(c, RQ_ERR_CONTEXT, "%d steps at position %d: past the capacity %d", n, s->len, s->cap);
-    int hd = m->head_dim;
-    if (!(fused_shape(m) && (hd == 128 || hd == 64 || hd == 32)) || gw_kv_att_q(s->kvt)) {
+    if (!(fused_shape(m) || fusedk_shape(m)) || gw_kv_att_q(s->kvt)) {
         for (int i = 0; i < n; i++) {
             if ((e = gw_decode_argmax(c, s, i ? tokens[i - 1] : token, &tokens[i])) != RQ_OK) return e;
         }
@@ -1072,11 +1091,11 @@ int gw_decode_greedy(RqCtx *c, RqSeq *s, int token, int n, int *tokens) {
     for (int i = 0; i < n; i++) {
         c->nev = 0;
         pf_mark(c, GW_PF_EMBED);
-        KCHK(gw_k_embed_q8(c->x, m->dim, (const uint8_t *)m->embd.codes, m->embd.scales, c->gtok_d + i, 1, st));
+        if ((e = embed_rows(c, c->gtok_d + i, 1)) != RQ_OK) return e;
         for (int l = 0; l < m->n_layers; l++)
             if ((e = fused_layer(c, l, s, p0 + i, c->gpos_d + i)) != RQ_OK) return e;
         pf_mark(c, GW_PF_CLS);
-        KCHK(gw_k_gemv1_norm(&m->cls, GW_GV_R_CLS, c->x, m->final_norm, c->logits_d, 0, 0, NULL, 0, st));
+        if ((e = fused_cls(c)) != RQ_OK) return e;
         pf_mark(c, -1);
         KCHK(gw_k_argmax(c->logits_d, m->vocab, m->vocab, 1, c->gtok_d + i + 1, c->argmax_scr, st));
         if (c->prof_on) { /* (profiling: each pass's intervals, as the passes of fw_pass) */
@@ -1225,7 +1244,7 @@ int gw_ctx_gemv_sweep(RqCtx *c, int reps, double *seconds, double *bytes, int *l
     const RqModel *m = c->m;
     if (reps < 1) return ctx_fail(c, RQ_ERR_ARG, "reps %d", reps);
     double b = 0;
-    int nl = 0, rc, fused = fused_shape(m);
+    int nl = 0, rc, fused = fused_shape(m), fusedk = fusedk_shape(m);
     hipStream_t s = c->stream;
     hipEvent_t e0, e1;
     HIPCHK(c, "hipEventCreate", hipEventCreate(&e0));
@@ -1244,13 +1263,24 @@ int gw_ctx_gemv_sweep(RqCtx *c, int reps, double *seconds, double *bytes, int *l
                                    last ? GW_GV_R_CLS : GW_GV_R_QKV, s));
                 continue;
             }
+            if (fusedk) {
+                GwGkIn in = { 0 };
+                in.x = c->x, in.nw = y->att_norm, in.part = c->part, in.pstride = c->pstride, in.hd = m->head_dim, in.nb = 1;
+                KCHK(gw_k_gemvk(GW_GK_NORM, y->qkv, 3, 0, &in, c->qkv, 0, s));
+                KCHK(gw_k_gemvk(GW_GK_COMBINE, &y->wo, 1, 0, &in, c->xb, 0, s));
+                KCHK(gw_k_gemvk(GW_GK_NORM, y->w13, 2, 1, &in, c->hb, 0, s));
+                in.x = c->hb;
+                KCHK(gw_k_gemvk(GW_GK_QF, &y->w2, 1, 0, &in, c->xb, 0, s));
+                continue;
+            }
             if ((rc = run_mm(c, y->qkv, y->nqkv, c->xq, c->xs, c->kmax, 1, c->qkv, c->ldqkv, 0)) != RQ_OK) return rc;
             if ((rc = run_mm(c, &y->wo, 1, c->xq, c->xs, c->kmax, 1, c->xb, m->dim, 0)) != RQ_OK) return rc;
             if ((rc = run_mm(c, y->w13, y->nw13, c->xq, c->xs, c->kmax, 1, c->hb, 2 * m->hidden, 0)) != RQ_OK) return rc;
             if ((rc = run_mm(c, &y->w2, 1, c->hq, c->hs, m->hidden, 1, c->xb, m->dim, 0)) != RQ_OK) return rc;
         }
-        if (fused) KCHK(gw_k_gemv1_norm(&m->cls, GW_GV_R_CLS, c->x, m->final_norm, c->logits_d, 0, 0, NULL, 0, s));
-        else if ((rc = run_mm(c, &m->cls, 1, c->xq, c->xs, c->kmax, 1, c->logits_d, m->vocab, 0)) != RQ_OK) return rc;
+        if (fused || fusedk) {
+            if ((rc = fused_cls(c)) != RQ_OK) return rc;
+        } else if ((rc = run_mm(c, &m->cls, 1, c->xq, c->xs, c->kmax, 1, c->logits_d, m->vocab, 0)) != RQ_OK) return rc;
     }
     HIPCHK(c, "hipEventRecord", hipEventRecord(e1, s));
     HIPCHK(c, "hipEventSynchronize", hipEventSynchronize(e1));
@@ -1269,7 +1299,7 @@ int gw_ctx_gemv_sweep(RqCtx *c, int reps, double *seconds, double *bytes, int *l
             }
     }
     b += gw_mat_file_bytes(&m->cls);
-    nl++;
+    nl = fusedk ? 4 * m->n_layers + 1 : nl + 1;
     if (seconds) *seconds = ms * 1e-3 / reps;
     if (bytes) *bytes = b;
     if (launches) *launches = nl;

@@ -1723,8 +1723,8 @@ __global__ __launch_bounds__(256) void k_embed_kq(float *__restrict__ x, int dim
     case GW_IQ3_XXS_R: embed_iq<GW_IQ3_XXS_R>(xo, dim, rb, bstride); return;
     case GW_IQ3_S_R: embed_iq<GW_IQ3_S_R>(xo, dim, rb, bstride); return;
     }
-    for (int i = threadIdx.x; i < dim; i += blockDim.x) {
-        int s = i >> 8, k = i & 255;
+    { // (block y: super-block y)
+        const int s = blockIdx.y, k = threadIdx.x, i = 256 * s + k;
         float y;
         if (type == GW_Q4_K || type == GW_Q5_K) {
             const uint8_t *b = rb + (size_t)s * bstride, *sc = b + 4;
@@ -2066,7 +2066,8 @@ int gw_k_kq_to_dev(const uint8_t *src, size_t nblk, int type, uint8_t *dst, hipS
 int gw_k_embed_kq(float *x, int dim, int type, const uint8_t *blocks, int bstride, const int *tok, int n, hipStream_t s) {
     hipEvent_t e0, e1;
     gw_take_launch_events(&e0, &e1);
-    hipExtLaunchKernelGGL(k_embed_kq, dim3(n), dim3(256), 0, s, e0, e1, 0, x, dim, type, blocks, bstride, tok);
+    const bool kq = type >= GW_Q2_K && type <= GW_Q6_K; // (a block per super-block: one row 8.9 -> EMB us; the i-quants a block per row)
+    hipExtLaunchKernelGGL(k_embed_kq, dim3(n, kq ? dim / 256 : 1), dim3(256), 0, s, e0, e1, 0, x, dim, type, blocks, bstride, tok);
     return (int)hipGetLastError();
 }
 

@@ -359,6 +359,322 @@ __global__ __launch_bounds__(NT) void k_gemv1(GvArgs a) {
     }
 }
 
+// ------------------------------------------------------------------------------------------ K-quant rows
+
+// The decode step's matmuls of a K-quant model, one row, with the producer of the activation in front as in k_gemv1 (the
+// same prologues; GV_Q takes the quantized row) and up to three matrices of different types per launch: a run of blocks
+// per matrix (about one block per CU in all), each block a run of the matrix's rows. A row is units: 16 bytes of nibbles
+// of Q4_K / Q5_K (32 weights: half of two neighbouring groups; the pair of lanes 2 i, 2 i + 1 the two halves), or of Q6_K
+// the 16 bytes of qh with both runs of ql (64 weights, half of four groups). The block's units (rows x units per row) are
+// dealt to its 512 threads in turn whatever K is, GK_D of them in flight per thread, the first ones issued before the
+// prologue's arithmetic. The activation row lies quantized in LDS, by unit: no lane holds any of it. Lane pairs add their
+// exact sums (DPP), each lane of a pair makes the terms of its own groups (k_gemv_mr's expressions: kquants.h:86-109,
+// :410-554) into LDS, and one lane per row folds the groups in order.
+// swiglu: the launch's rows are pairs (w1 row, w3 row); the fold's two values of a pair give swiglu_ref(h, h2).
+// What bounds it: the launch's edges and the prologue, as k_gemv1 (a 4B layer's matrices are 9 - 28 MB). The layer's
+// matmuls, norms, SwiGLU, rope and combine as thirteen launches before: 100 us per layer at 701 positions -> GK_LAYER
+#define GK_T 512
+#define GK_LDS (100 << 10) // terms of a block's rows: at most this; more rows (the classifier) are folded in runs
+struct GkSeg {
+    const uint8_t *W, *W2; // (W2: swiglu, the second matrix of the pairs)
+    int type, bstride, rows, b0, rpb, col; // rows (pairs) of the matrix, its first block, rows per block, out's column
+};
+struct GkArgs {
+    GkSeg seg[3];
+    int nseg, K, swiglu, mode, run; // run: rows folded at a time (run x units per row: whole rounds of the block, or all its rows)
+    const int8_t *xq;
+    const float *xs, *x, *nw, *part;
+    int pstride, hd, nb;
+    float inv_k;
+    float *out;
+};
+
+template <int TYPE>
+struct GkUnit { // a unit's loads
+    uint4 a, b, c, hd;
+    uint32_t d;
+    __device__ __forceinline__ void load(const uint8_t *w, int u, int bstride) { // (w: the row)
+        auto ld = [](const uint8_t *p) __attribute__((always_inline)) -> uint4 {
+            typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+            return __builtin_bit_cast(uint4, __builtin_nontemporal_load((const u4 *)p));
+        };
+        if constexpr (TYPE == GW_Q6_K) { // (u: super-block u / 4, half n = u / 2 % 2, half-groups h = u % 2)
+            const uint8_t *o = w + (u >> 2) * bstride, *p = o + 64 * (u >> 1 & 1) + 16 * (u & 1);
+            a = ld(p);
+            b = ld(p + 32);
+            c = ld(o + 128 + 32 * (u >> 1 & 1) + 16 * (u & 1));
+            hd = ld(o + 192);
+            d = __builtin_nontemporal_load((const uint32_t *)(o + 208));
+        } else { // (u: super-block u / 8, groups 2 i, 2 i + 1 with i = u / 2 % 4, half-groups h = u % 2)
+            const uint8_t *o = w + (u >> 3) * bstride;
+            a = ld(o + (TYPE == GW_Q5_K ? 48 : 16) + 16 * (u & 7));
+            hd = ld(o);
+            if constexpr (TYPE == GW_Q5_K) b = ld(o + 16 + 16 * (u & 1));
+        }
+    }
+};
+__device__ __forceinline__ int gk_pair(int x) { return __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, true); } // lane ^ 1's value
+__device__ __forceinline__ int gk_dot(const uint4 w, const int4 x) {
+    int s = __builtin_amdgcn_sdot4((int)w.x, x.x, 0, false);
+    s = __builtin_amdgcn_sdot4((int)w.y, x.y, s, false);
+    s = __builtin_amdgcn_sdot4((int)w.z, x.z, s, false);
+    return __builtin_amdgcn_sdot4((int)w.w, x.w, s, false);
+}
+
+// the terms of unit u of a row into T (the row's groups); xc: the half-groups' codes, those of even groups by unit pair,
+// then those of odd ones (K / 32 each); hs: their sums, alike; xs, xf per group
+template <int TYPE>
+__device__ __forceinline__ void gk_terms(const GkUnit<TYPE> &U, int u, int K, const int4 *xc, const int *hs, const float *xs,
+                                         const float *xf, float *T, bool in) {
+    const bool odd = threadIdx.x & 1; // (units per row are even, so are a block's threads: u % 2 == threadIdx.x % 2)
+    const int H2 = K >> 5;
+    if constexpr (TYPE == GW_Q6_K) {
+        const int base = 4 * (u >> 1) + (u & 1);
+        auto code = [&](const uint4 lo, int sl, int sh) __attribute__((always_inline)) -> uint4 { // (sh: qh's shift, left if > 0)
+            const uint32_t l[4] = { lo.x, lo.y, lo.z, lo.w }, h[4] = { U.c.x, U.c.y, U.c.z, U.c.w };
+            uint32_t q[4];
+            #pragma unroll
+            for (int e = 0; e < 4; e++) q[e] = ((l[e] >> sl) & 0x0F0F0F0Fu) | ((sh >= 0 ? h[e] << sh : h[e] >> -sh) & 0x30303030u);
+            return make_uint4(q[0], q[1], q[2], q[3]);
+        };
+        const uint32_t w0 = (u >> 1 & 1) ? U.hd.z : U.hd.x, w1 = (u >> 1 & 1) ? U.hd.w : U.hd.y;
+        const int s8 = 8 * (u & 1);
+        const int sc[4] = { (int)(int8_t)(w0 >> s8), (int)(int8_t)(w0 >> (16 + s8)), (int)(int8_t)(w1 >> s8), (int)(int8_t)(w1 >> (16 + s8)) };
+        const uint4 q[4] = { code(U.a, 0, 4), code(U.b, 0, 2), code(U.a, 4, 0), code(U.b, 4, -2) };
+        int I[4];
+        #pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const int k = (p & 1) * H2 + base + (p & 2);
+            I[p] = sc[p] * (gk_dot(q[p], xc[k]) - 32 * hs[k]);
+        }
+        const int r0 = gk_pair(odd ? I[0] : I[2]), r1 = gk_pair(odd ? I[1] : I[3]);
+        const int i0 = (odd ? I[2] : I[0]) + r0, i1 = (odd ? I[3] : I[1]) + r1, g = 4 * (u >> 1) + (odd ? 2 : 0);
+        const float d = h2f((uint16_t)(U.d & 0xffffu)), t0 = (d * xs[g]) * (float)i0, t1 = (d * xs[g + 1]) * (float)i1;
+        if (in) *(float2 *)(T + g) = make_float2(t0, t1);
+    } else {
+        const int i = (u >> 1) & 3;
+        const uint32_t w[4] = { U.a.x, U.a.y, U.a.z, U.a.w }, hb[4] = { U.b.x, U.b.y, U.b.z, U.b.w };
+        uint32_t lo[4], hi[4];
+        #pragma unroll
+        for (int e = 0; e < 4; e++) {
+            lo[e] = w[e] & 0x0F0F0F0Fu;
+            hi[e] = (w[e] >> 4) & 0x0F0F0F0Fu;
+            if constexpr (TYPE == GW_Q5_K) {
+                const uint32_t z = hb[e] >> (2 * i);
+                lo[e] |= (z & 0x01010101u) << 4;
+                hi[e] |= (z & 0x02020202u) << 3;
+            }
+        }
+        const int sl = gk_dot(make_uint4(lo[0], lo[1], lo[2], lo[3]), xc[u]), sh = gk_dot(make_uint4(hi[0], hi[1], hi[2], hi[3]), xc[H2 + u]);
+        const int r = gk_pair(odd ? sl : sh), I = (odd ? sh : sl) + r, j = 2 * i + (odd ? 1 : 0), jb = 8 * (j & 3), g = 2 * (u >> 1) + (odd ? 1 : 0);
+        const uint32_t y = U.hd.y >> jb, z = U.hd.z >> jb, x = U.hd.w >> jb;
+        const int scj = (int)(j < 4 ? y & 63u : (x & 15u) | ((y >> 6) & 3u) << 4), mj = (int)(j < 4 ? z & 63u : ((x >> 4) & 15u) | ((z >> 6) & 3u) << 4);
+        const float f0 = h2f((uint16_t)(U.hd.x & 0xffffu)) * (float)scj, f1 = h2f((uint16_t)(U.hd.x >> 16)) * (float)mj;
+        const float a = (f0 * xs[g]) * (float)I, b = f1 * xf[g];
+        if (in) T[g] = a - b;
+    }
+}
+
+// the block's rows of one matrix (or pairs of two): loads of the first D units, then `pro` (the prologue), then the units in
+// turn, a fold every a.run rows
+template <int TYPE, int D, typename F>
+__device__ __forceinline__ void gk_rows(const GkArgs &a, const GkSeg &g, int blk, float *T, const int4 *xc, const int *hs, const float *xs,
+                                        const float *xf, F pro) {
+    const int K = a.K, G = K >> 5, PS = (G + 7) & ~3, P = TYPE == GW_Q6_K ? K >> 6 : K >> 5, rowb = (K >> 8) * g.bstride;
+    const int t = threadIdx.x, f0 = blk * g.rpb, nr = g.rows - f0 < g.rpb ? g.rows - f0 : g.rpb, nrow = a.swiglu ? 2 * nr : nr;
+    const int q = GK_T / P, rr = GK_T - q * P, tot = nrow * P, rounds = (tot + GK_T - 1) / GK_T, per = a.run * P / GK_T;
+    const uint8_t *w1 = g.W + (size_t)f0 * rowb, *w2 = a.swiglu ? g.W2 + (size_t)f0 * rowb - (size_t)nr * rowb : w1; // (rows from nr on)
+    GkUnit<TYPE> U[D];
+    int lrow = t / P, lu = t - lrow * P, row = lrow, u = lu; // (the next unit to load, the next to use)
+    auto load = [&](GkUnit<TYPE> &x) __attribute__((always_inline)) {
+        // (pairs: rows 0 .. nr - 1 of the first matrix, then those of the second; past the last row its loads again)
+        const int r = lrow < nrow ? lrow : nrow - 1;
+        x.load((r < nr ? w1 : w2) + (size_t)(uint32_t)(r * rowb), lu, g.bstride);
+        lrow += q, lu += rr;
+        if (lu >= P) lu -= P, lrow++;
+    };
+    #pragma unroll
+    for (int d = 0; d < D; d++) load(U[d]);
+    pro();
+    int r0 = 0, in_run = 0; // (the run's first row, its rounds so far)
+    auto step = [&](GkUnit<TYPE> &x, int it) __attribute__((always_inline)) {
+        const bool in = row < nrow;
+        gk_terms<TYPE>(x, u, K, xc, hs, xs, xf, T + (in ? row - r0 : 0) * PS, in);
+        row += q, u += rr;
+        if (u >= P) u -= P, row++;
+        load(x);
+        if (++in_run == per || it + 1 == rounds) {
+            __syncthreads();
+            const int n = nrow - r0 < a.run ? nrow - r0 : a.run;
+            float v = t < n ? gv_fold(T + (size_t)t * PS, G) : 0.0f;
+            if (a.swiglu) { // (all rows in one run: lane nr + i holds the second matrix's row i)
+                __syncthreads();
+                if (t >= nr && t < n) T[t - nr] = v;
+                __syncthreads();
+                if (t < nr) a.out[g.col + f0 + t] = swiglu_ref(v, T[t]);
+            } else if (t < n) {
+                float *o = a.out + g.col + f0 + r0 + t;
+                *o = a.mode == 1 ? *o + v : v;
+            }
+            __syncthreads();
+            r0 += a.run;
+            in_run = 0;
+        }
+    };
+    for (int it = 0; it < rounds; it += D) {
+        #pragma unroll
+        for (int d = 0; d < D; d++)
+            if (it + d < rounds) step(U[d], it + d);
+    }
+}
+
+template <int PRO>
+__global__ __launch_bounds__(GK_T) void k_gemvk(GkArgs a) {
+    extern __shared__ __align__(16) uint8_t gk_lds[];
+    const int K = a.K, G = K >> 5, H = K >> 4, t = threadIdx.x;
+    int4 *const xc = (int4 *)gk_lds;               // K bytes
+    int *const hs = (int *)(gk_lds + K);           // H sums
+    float *const xs = (float *)(hs + H), *const xf = xs + G, *const T = xf + G; // G, G, then the terms (and GV_NORM's row)
+    int si = 0;
+    #pragma unroll
+    for (int i = 1; i < 3; i++)
+        if (i < a.nseg && (int)blockIdx.x >= a.seg[i].b0) si = i;
+    const GkSeg g = a.seg[si];
+    // the prologue's loads: 16-value chunks t and (QF) t + GK_T of the row
+    constexpr int NCK = PRO == GV_QF ? 2 : 1;
+    float4 p0[NCK][4], p1[4];
+    float2 po[PRO == GV_COMBINE ? GV_NBMAX : 1][8];
+    float pm[GV_NBMAX], pl[GV_NBMAX];
+    int4 xv;
+    float xsv = 0.0f;
+    const int j0 = t < H ? t : H - 1, nb = PRO == GV_COMBINE ? a.nb : 1;
+    if constexpr (PRO == GV_Q) {
+        xv = *(const int4 *)(a.xq + 16 * j0);
+        xsv = a.xs[j0 >> 1];
+    } else if constexpr (PRO == GV_COMBINE) {
+        const int st = a.hd + 2, e0 = 16 * j0, i0 = e0 % a.hd;
+        const float *pb = a.part + (size_t)(e0 / a.hd) * a.pstride + i0;
+        #pragma unroll
+        for (int b = 0; b < GV_NBMAX; b++) {
+            const float *q = pb + (b < nb ? b : nb - 1) * st;
+            #pragma unroll
+            for (int u = 0; u < 8; u++) po[b][u] = ((const float2 *)q)[u];
+            pm[b] = q[a.hd - i0];
+            pl[b] = q[a.hd - i0 + 1];
+        }
+    } else {
+        #pragma unroll
+        for (int c = 0; c < NCK; c++) {
+            const int j = t + GK_T * c < H ? t + GK_T * c : H - 1;
+            #pragma unroll
+            for (int u = 0; u < 4; u++) p0[c][u] = ((const float4 *)(a.x + 16 * j))[u];
+        }
+        if constexpr (PRO == GV_NORM) {
+            #pragma unroll
+            for (int u = 0; u < 4; u++) p1[u] = ((const float4 *)(a.nw + 16 * j0))[u];
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // chunk j's codes, half-group sum and (even lanes) its group's scale and xs (float) sum into LDS
+    auto put = [&](int j, const int4 q, float s) __attribute__((always_inline)) {
+        int sx = __builtin_amdgcn_sdot4(q.x, 0x01010101, 0, false);
+        sx = __builtin_amdgcn_sdot4(q.y, 0x01010101, sx, false);
+        sx = __builtin_amdgcn_sdot4(q.z, 0x01010101, sx, false);
+        sx = __builtin_amdgcn_sdot4(q.w, 0x01010101, sx, false);
+        const int full = sx + gk_pair(sx);
+        if (j < H) {
+            const int k = ((j >> 1) & 1) * G + 2 * (j >> 2) + (j & 1);
+            xc[k] = q;
+            hs[k] = sx;
+            if (!(j & 1)) xs[j >> 1] = s, xf[j >> 1] = s * (float)full;
+        }
+    };
+    auto pro = [&]() __attribute__((always_inline)) {
+        if constexpr (PRO == GV_Q) {
+            put(t, xv, xsv);
+        } else {
+            float v[16];
+            if constexpr (PRO == GV_NORM) { // (k_gemv1's: the row in the chains' layout, the 16 chains, the tree)
+                const int n4 = K >> 6, NF = rms_nf(n4), LS = 4 * NF + 4;
+                if (t < H) {
+                    #pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        T[(4 * u + 0) * LS + t] = p0[0][u].x;
+                        T[(4 * u + 1) * LS + t] = p0[0][u].y;
+                        T[(4 * u + 2) * LS + t] = p0[0][u].z;
+                        T[(4 * u + 3) * LS + t] = p0[0][u].w;
+                    }
+                }
+                if (NF > n4)
+                    for (int z = t; z < 16 * (NF - n4); z += GK_T)
+                        ((float4 *)T)[(z / (NF - n4)) * (NF + 1) + n4 + z % (NF - n4)] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                __syncthreads();
+                if (t < 64) {
+                    const float r = rms_scale_t(T, K);
+                    if (t == 0) xs[0] = r;
+                }
+                __syncthreads();
+                const float r = xs[0];
+                __syncthreads(); // (xs[0] is the first group's scale next)
+                #pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    v[4 * u + 0] = (p1[u].x * p0[0][u].x) * r;
+                    v[4 * u + 1] = (p1[u].y * p0[0][u].y) * r;
+                    v[4 * u + 2] = (p1[u].z * p0[0][u].z) * r;
+                    v[4 * u + 3] = (p1[u].w * p0[0][u].w) * r;
+                }
+            } else if constexpr (PRO == GV_COMBINE) { // (att_combine, as k_gemv1)
+                if (nb == 1) {
+                    const float inv = 1.0f / pl[0];
+                    #pragma unroll
+                    for (int u = 0; u < 8; u++) v[2 * u] = po[0][u].x * inv, v[2 * u + 1] = po[0][u].y * inv;
+                } else {
+                    float M = pm[0];
+                    #pragma unroll
+                    for (int b = 1; b < GV_NBMAX; b++)
+                        if (b < nb) M = pm[b] > M ? pm[b] : M;
+                    float cb[GV_NBMAX], L = 0.0f;
+                    #pragma unroll
+                    for (int b = 0; b < GV_NBMAX; b++)
+                        if (b < nb) {
+                            cb[b] = exp_att(pm[b] - M);
+                            L = __builtin_fmaf(cb[b], pl[b], L);
+                        }
+                    const float inv = 1.0f / L;
+                    #pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        float a0 = 0.0f, a1 = 0.0f;
+                        #pragma unroll
+                        for (int b = 0; b < GV_NBMAX; b++)
+                            if (b < nb) {
+                                a0 = __builtin_fmaf(cb[b], po[b][u].x, a0);
+                                a1 = __builtin_fmaf(cb[b], po[b][u].y, a1);
+                            }
+                        v[2 * u] = a0 * inv;
+                        v[2 * u + 1] = a1 * inv;
+                    }
+                }
+            }
+            #pragma unroll
+            for (int c = 0; c < NCK; c++) {
+                if constexpr (PRO == GV_QF) {
+                    #pragma unroll
+                    for (int u = 0; u < 4; u++) v[4 * u] = p0[c][u].x, v[4 * u + 1] = p0[c][u].y, v[4 * u + 2] = p0[c][u].z, v[4 * u + 3] = p0[c][u].w;
+                }
+                int4 q;
+                float s;
+                gv_quant16(v, q, s);
+                put(t + GK_T * c, q, s);
+            }
+        }
+        __syncthreads();
+    };
+    const int blk = (int)blockIdx.x - g.b0;
+    if (g.type == GW_Q4_K) gk_rows<GW_Q4_K, 4>(a, g, blk, T, xc, hs, xs, xf, pro);
+    else if (g.type == GW_Q5_K) gk_rows<GW_Q5_K, 3>(a, g, blk, T, xc, hs, xs, xf, pro);
+    else gk_rows<GW_Q6_K, 3>(a, g, blk, T, xc, hs, xs, xf, pro);
+}
+
 extern "C" {
 
 // the matmul out[row] (+)= W row . act, act = the prologue's quantized row; R weight rows per block (4, 8 or 16)
@@ -475,6 +791,74 @@ int gw_k_gemv1_combine(const GwMat *w, int R, const float *part, int pstride, in
     a.W = w->codes, a.WS = w->scales, a.nrows = w->rows, a.K = w->cols, a.part = part, a.pstride = pstride, a.hd = hd;
     a.nb = nb, a.out = out, a.mode = mode;
     return gv_launch(GV_COMBINE, R, a, nx, nR, s);
+}
+
+static int gk_plan(int pro, const GwMat *w, int nmat, int swiglu, GkArgs *a, int *nblocks, size_t *lds) {
+    /* the launch of w[0 .. nmat - 1] (0), or hipErrorInvalidValue where k_gemvk does not take it */
+    const int K = w[0].cols, G = K / 32, PS = (G + 7) & ~3, cus = gw_device_cus(), ns = swiglu ? 1 : nmat;
+    if (nmat < 1 || nmat > 3 || K < 256 || K % 256 || K > (pro == GV_QF ? 32 * GK_T : pro == GV_Q ? 16 * GK_T : 4096) ||
+        (swiglu && (nmat != 2 || w[0].type != w[1].type || w[0].rows != w[1].rows)))
+        return (int)hipErrorInvalidValue;
+    size_t bytes[3], total = 0;
+    for (int i = 0; i < nmat; i++) {
+        if ((w[i].type != GW_Q4_K && w[i].type != GW_Q5_K && w[i].type != GW_Q6_K) || w[i].cols != K || ((uintptr_t)w[i].blocks & 15))
+            return (int)hipErrorInvalidValue;
+        bytes[i] = (size_t)w[i].rows * (K / 256) * w[i].bstride;
+        if (i < ns) total += bytes[i];
+    }
+    int b0 = 0, col = 0, maxr = 0;
+    for (int i = 0; i < ns; i++) { // (each matrix its share of the CUs by bytes, a block one row at least)
+        GkSeg *g = &a->seg[i];
+        int nblk = (int)((bytes[i] * cus + total / 2) / total);
+        nblk = nblk < 1 ? 1 : nblk > w[i].rows ? w[i].rows : nblk;
+        g->W = w[i].blocks, g->W2 = swiglu ? w[1].blocks : NULL, g->type = w[i].type, g->bstride = w[i].bstride, g->rows = w[i].rows;
+        g->rpb = (w[i].rows + nblk - 1) / nblk;
+        nblk = (w[i].rows + g->rpb - 1) / g->rpb;
+        g->b0 = b0, g->col = col;
+        b0 += nblk, col += w[i].rows;
+        maxr = g->rpb > maxr ? g->rpb : maxr;
+        if ((size_t)2 * g->rpb * (K / 256) * g->bstride >= ((size_t)1 << 31)) return (int)hipErrorInvalidValue;
+    }
+    const int rows = swiglu ? 2 * maxr : maxr, most = GK_LDS / (PS * 4) < GK_T ? GK_LDS / (PS * 4) : GK_T;
+    if (rows <= most) {
+        a->run = rows + GK_T; // (one run: more rounds than there are)
+    } else { // (runs of rows whose units, K / 64 each at least, are whole rounds of the block's threads)
+        int step = 1;
+        while ((size_t)step * (K / 64) % GK_T) step *= 2;
+        a->run = most / step * step;
+        if (swiglu || a->run < 1) return (int)hipErrorInvalidValue;
+    }
+    const size_t terms = (size_t)(rows <= most ? rows : a->run) * PS * 4, row = pro == GV_NORM ? (size_t)16 * (4 * rms_nf(K / 64) + 4) * 4 : 0;
+    a->nseg = ns, a->K = K, a->swiglu = swiglu, a->inv_k = 1.0f / (float)K;
+    *nblocks = b0;
+    *lds = (size_t)K + K / 16 * 4 + 2 * G * 4 + (terms > row ? terms : row);
+    return 0;
+}
+
+int gw_k_gemvk_ok(int pro, const GwMat *w, int nmat, int swiglu) {
+    GkArgs a = {};
+    int nb;
+    size_t lds;
+    return gk_plan(pro, w, nmat, swiglu, &a, &nb, &lds) == 0;
+}
+
+int gw_k_gemvk(int pro, const GwMat *w, int nmat, int swiglu, const GwGkIn *in, float *out, int mode, hipStream_t s) {
+    GkArgs a = {};
+    int b0;
+    size_t lds;
+    if (gk_plan(pro, w, nmat, swiglu, &a, &b0, &lds) || (pro == GV_COMBINE && (in->hd % 16 || in->nb < 1 || in->nb > GV_NBMAX)))
+        return (int)hipErrorInvalidValue;
+    a.mode = mode, a.xq = in->xq, a.xs = in->xs, a.x = in->x, a.nw = in->nw, a.part = in->part;
+    a.pstride = in->pstride, a.hd = in->hd, a.nb = in->nb, a.out = out;
+    hipEvent_t e0, e1;
+    gw_take_launch_events(&e0, &e1);
+#define GK_L(PP) hipExtLaunchKernelGGL((k_gemvk<PP>), dim3(b0), dim3(GK_T), (uint32_t)lds, s, e0, e1, 0, a)
+    if (pro == GV_Q) GK_L(GV_Q);
+    else if (pro == GV_NORM) GK_L(GV_NORM);
+    else if (pro == GV_QF) GK_L(GV_QF);
+    else GK_L(GV_COMBINE);
+#undef GK_L
+    return (int)hipGetLastError();
 }
 
 } // extern "C"

@@ -427,6 +427,19 @@ int gw_k_gemv1_qf(const GwMat *w, int R, const float *x, float *out, int mode, c
 int gw_k_gemv1_combine(const GwMat *w, int R, const float *part, int pstride, int hd, int nb, float *out, int mode,
                        const GwMat *nx, int nR, hipStream_t s);
 
+/* the one-row matmuls of a K-quant model (k_gemvk): w[0 .. nmat - 1] of one width (Q4_K, Q5_K, Q6_K; gw_k_gemvk_ok: whether it takes them) side by
+ * side in out (mode 1: out += ), the activation made by the prologue pro: GW_GK_Q the quantized row xq / xs, GW_GK_NORM
+ * rmsnorm of x with weights nw (K <= 4096), GW_GK_QF the fp32 row x (K <= 16384), GW_GK_COMBINE the attention partials (K <=
+ * 4096, nb <= GW_GV_NBMAX). swiglu: w[0] and w[1] are w1 and w3, out the SwiGLU of their rows */
+typedef struct {
+    const int8_t *xq;
+    const float *xs, *x, *nw, *part;
+    int pstride, hd, nb;
+} GwGkIn;
+enum { GW_GK_Q = 0, GW_GK_NORM = 1, GW_GK_QF = 2, GW_GK_COMBINE = 3 }; /* (gw_gemv.hip's prologues) */
+int gw_k_gemvk_ok(int pro, const GwMat *w, int nmat, int swiglu);
+int gw_k_gemvk(int pro, const GwMat *w, int nmat, int swiglu, const GwGkIn *in, float *out, int mode, hipStream_t s);
+
 /* per-launch kernel timing (gw_ctx_kernel_timing): gw_time_next_launch(a, b) makes the next matmul launch (k_gemv1,
  * k_gemm_q8, k_gemv_mr) record its own start and stop in events a and b (hipExtLaunchKernel's events: the
  * dispatch's timestamps, no extra packets on the stream); each launcher takes the pair once (gw_take_launch_events) */

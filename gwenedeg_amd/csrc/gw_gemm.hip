@@ -2066,7 +2066,7 @@ int gw_k_kq_to_dev(const uint8_t *src, size_t nblk, int type, uint8_t *dst, hipS
 int gw_k_embed_kq(float *x, int dim, int type, const uint8_t *blocks, int bstride, const int *tok, int n, hipStream_t s) {
     hipEvent_t e0, e1;
     gw_take_launch_events(&e0, &e1);
-    const bool kq = type >= GW_Q2_K && type <= GW_Q6_K; // (a block per super-block: one row 8.9 -> EMB us; the i-quants a block per row)
+    const bool kq = type >= GW_Q2_K && type <= GW_Q6_K; // (a block per super-block: one row 8.9 -> 3.0 us; the i-quants a block per row)
     hipExtLaunchKernelGGL(k_embed_kq, dim3(n, kq ? dim / 256 : 1), dim3(256), 0, s, e0, e1, 0, x, dim, type, blocks, bstride, tok);
     return (int)hipGetLastError();
 }

@@ -379,15 +379,17 @@ int gw_k_attn_q(const void *items, int nitems, const float *qkv, int ldqkv, int 
                 hipStream_t s);
 /* the rows of quantized caches: o = D H o' / hd from the combined attention att (n rows of nh hd), quantized into aq / as */
 int gw_k_unrot_quant(const float *att, int n, int nh, int hd, const int *kvt, int8_t *aq, float *as, int ldq, hipStream_t s);
+/* the attention partials of items on the 16-bit caches (kbf: bf16); narrow: every item one row of at most 4 query vectors */
 int gw_k_attn_part(const void *items, int nitems, const float *qkv, int ldqkv, int nh, int nkv, int hd, float scale,
                    const int *pos, uint16_t *const *kc, uint16_t *const *vc, float *part, int pstride, int kbf, int narrow, hipStream_t s);
+int gw_device_cus(void); /* the device's compute units */
 /* the one-row pass's attention with its QK-norm, RoPE and K / V store (hd 32, 64 or 128; pos: the row's position;
  * kl / vl: its sequence's K / V cache of the layer) */
-int gw_device_cus(void);
 int gw_k_attn_decode(const float *qkv, int nh, int nkv, int hd, float scale, const float *qn, const float *kn, const float *rope,
                      int pos, uint16_t *kl, uint16_t *vl, float *part, int pstride, int kbf, hipStream_t s);
-/* the rows' attention from their key blocks' partials, quantized for wo (nbmax: the most key blocks of any row) */
+/* n floats from the device to pinned host memory by a kernel (both 16-byte aligned) */
 int gw_k_copy_out(float *dst, const float *src, size_t n, hipStream_t s);
+/* the rows' attention from their key blocks' partials, quantized for wo (nbmax: the most key blocks of any row) */
 int gw_k_attn_combine_quant(const float *part, int pstride, int nh, int hd, const int *pos, int n, int nbmax, int8_t *aq,
                             float *as, int ldq, float *att_out, hipStream_t s);
 /* hb row: [h (H) | h2 (H)] (il = 0) or blocks of il h then il h2 (w1 / w3 rows interleaved by il) */

@@ -732,7 +732,12 @@ typedef struct {
 static int run_mm(RqCtx *c, const GwMat *w, int nmat, const int8_t *xq, const float *xs, int ldx, int M, float *out, int ldo,
                   int mode) {
     /* the matrices side by side in out's columns; two neighbours of one K-quant type share a launch where the kernel
-     * allows (gw_k_matmul2) */
+     * allows (gw_k_matmul2), and a layer's q, k and v (gw_k_matmul3) */
+    if (nmat == 3) {
+        const int e = gw_k_matmul3(w, xq, xs, ldx, M, out, ldo, mode, c->stream);
+        if (e > 0) return ctx_fail(c, RQ_ERR_STATE, "matmul launch failed (%d x %d, type %d)", w[0].rows, w[0].cols, w[0].type);
+        if (!e) return RQ_OK;
+    }
     for (int i = 0, col = 0; i < nmat;) {
         if (i) kt_next(c, c->kt_cur); /* (the first launch's pair is set by the class mark) */
         int two = i + 1 < nmat, e = -1;

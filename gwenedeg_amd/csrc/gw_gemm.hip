@@ -923,24 +923,32 @@ __device__ __forceinline__ void kq32_terms(const i32x16 &I, const i32x16 &I1, co
         Tq[e * 64 + lane] = term;
     }
 }
+template <int TYPE>
+constexpr int SK_WST = TYPE == GW_Q4_K ? 160 : 240;             // LDS bytes per weight row (bstride + 16)
 template <int TYPE, int NQR, int SB>
-__global__ __launch_bounds__(SK_T * SB, SB == 1 ? 2 : 1) void k_gemm_kq32(SkMats mats, int bstride, int K,
-                                                                          const int8_t *__restrict__ X,
-                                                                          const float *__restrict__ XS, int ldx, int M,
-                                                                          float *out, int ldo, int mode) {
-    constexpr int WST = TYPE == GW_Q4_K ? 160 : 240;            // LDS bytes per weight row (bstride + 16)
+struct SkLds {
+    alignas(16) float Tl[8 * SB][NQR * 256];                    // term of group g of super-block b (row 8 b + g)
+    alignas(16) uint8_t Ws[2][SB][32 * SK_WST<TYPE>];
+    alignas(16) uint8_t Xs[2][SB][32 * SK_XR];
+    alignas(16) float xsl[2][SB][8][32];                        // [super-block][group][m]
+};
+template <int TYPE, int NQR, int SB>
+__device__ __forceinline__ void kq32_block(SkLds<TYPE, NQR, SB> &lds, int bx, const SkMats &mats, int bstride, int K,
+                                           const int8_t *__restrict__ X, const float *__restrict__ XS, int ldx, int M, float *out,
+                                           int ldo, int mode) { // (bx: the block among those of mats)
+    constexpr int WST = SK_WST<TYPE>;
     constexpr int PW = TYPE == GW_Q4_K ? GW_Q4K_BYTES / 16 : GW_Q6K_DEV / 16; // 16-byte pieces per weight row
     constexpr int PARTS = 4 / NQR, NO = NQR * 256, NT = SK_T * SB; // blocks per tile, outputs per block, threads
-    __shared__ __align__(16) float Tl[8 * SB][NO];              // term of group g of super-block b (row 8 b + g)
-    __shared__ __align__(16) uint8_t Ws[2][SB][32 * WST];
-    __shared__ __align__(16) uint8_t Xs[2][SB][32 * SK_XR];
-    __shared__ __align__(16) float xsl[2][SB][8][32];           // [super-block][group][m]
+    auto &Tl = lds.Tl;
+    auto &Ws = lds.Ws;
+    auto &Xs = lds.Xs;
+    auto &xsl = lds.xsl;
     // wave wv: group w = wv % 8 of super-block sb = wv / 8 of the step; thread t stages super-block ts = t / SK_T
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6, w = wv & 7, sb = wv >> 3, hi = lane >> 5, r32 = lane & 31;
     const int tt = t & (SK_T - 1), ts = t / SK_T;
-    const int mi = blockIdx.x >= mats.nb1;
+    const int mi = bx >= mats.nb1;
     // block b of its matrix: XCD b % 8, then (b / 8) % PARTS its quads, tile 8 (b / 8 / PARTS) + b % 8
-    const int bl = blockIdx.x - (mi ? mats.nb1 : 0), part = (bl >> 3) % PARTS, q0 = part * NQR;
+    const int bl = bx - (mi ? mats.nb1 : 0), part = (bl >> 3) % PARTS, q0 = part * NQR;
     const int n0 = (((bl >> 3) / PARTS) * 8 + (bl & 7)) * 32, N = mats.N[mi], S = K >> 8;
     if (n0 >= N || 8 * q0 >= M) return; // (the grid's padding to 8 tiles; quads past the last activation row)
     const int S2 = (S + SB - 1) / SB; // (steps of SB super-blocks)
@@ -1110,6 +1118,29 @@ __global__ __launch_bounds__(SK_T * SB, SB == 1 ? 2 : 1) void k_gemm_kq32(SkMats
             *po = mode == 1 ? *po + v : v;
         }
     }
+}
+
+template <int TYPE, int NQR, int SB>
+__global__ __launch_bounds__(SK_T * SB, SB == 1 ? 2 : 1) void k_gemm_kq32(SkMats mats, int bstride, int K,
+                                                                          const int8_t *__restrict__ X,
+                                                                          const float *__restrict__ XS, int ldx, int M,
+                                                                          float *out, int ldo, int mode) {
+    __shared__ SkLds<TYPE, NQR, SB> lds;
+    kq32_block<TYPE, NQR, SB>(lds, (int)blockIdx.x, mats, bstride, K, X, XS, ldx, M, out, ldo, mode);
+}
+
+// two matrices of type TA (mats; blocks [0, bv)) and a third of type TV (mv; blocks from bv on) of one width: a layer's
+// q, k and v. v has few tiles (1,024 rows: 32 blocks) and as a launch of its own took as long as q and k beside it
+template <int TA, int TV>
+__global__ __launch_bounds__(SK_T, 2) void k_gemm_kq32_3(SkMats mats, SkMats mv, int bv, int bstride, int bstride_v, int K,
+                                                         const int8_t *__restrict__ X, const float *__restrict__ XS, int ldx,
+                                                         int M, float *out, int ldo, int mode) {
+    constexpr size_t LA = sizeof(SkLds<TA, 4, 1>), LV = sizeof(SkLds<TV, 4, 1>);
+    __shared__ __align__(16) uint8_t lds[LA > LV ? LA : LV];
+    if ((int)blockIdx.x < bv)
+        kq32_block<TA, 4, 1>(*(SkLds<TA, 4, 1> *)lds, (int)blockIdx.x, mats, bstride, K, X, XS, ldx, M, out, ldo, mode);
+    else
+        kq32_block<TV, 4, 1>(*(SkLds<TV, 4, 1> *)lds, (int)blockIdx.x - bv, mv, bstride_v, K, X, XS, ldx, M, out, ldo, mode);
 }
 
 // Q4_K GEMM of many tiles (prefill): k_gemm_q8l's 64 x 128 blocks (8 waves of 32 x 32, the XCD-aware order) and its copies
@@ -2274,6 +2305,32 @@ int gw_k_matmul2(const GwMat *a, const GwMat *b, int col_b, const int8_t *xq, co
     if (kq32_takes(a, M) && kq32_takes(b, M) && a->type == b->type && a->cols == b->cols && a->bstride == b->bstride)
         return launch_kq32(a, b, col_b, xq, xs, ldx, M, out, ldo, mode, s);
     return -1;
+}
+
+int gw_k_matmul3(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int M, float *out, int ldo, int mode, hipStream_t s) {
+    /* w[0], w[1] (of one type) and w[2], side by side in out's columns, in one launch where k_gemm_kq32 takes all three; else
+     * -1 and nothing launched. Every block is resident at once: w[0] and w[1] have at most a tile per CU (more go to
+     * k_gemm_kqt), w[2] too, and a CU holds two blocks */
+    for (int i = 0; i < 3; i++)
+        if (!kq32_takes(&w[i], M) || w[i].cols != w[0].cols) return -1;
+    if (w[0].type != w[1].type || w[0].bstride != w[1].bstride || (w[0].type == GW_Q6_K && w[2].type != GW_Q6_K) || g_kq16 || g_kq32_nqr ||
+        g_kq32_sb || kql_takes(&w[0], w[0].rows + w[1].rows, xq, xs, ldx, M) || kql_takes(&w[2], w[2].rows, xq, xs, ldx, M))
+        return -1;
+    hipEvent_t e0, e1;
+    gw_take_launch_events(&e0, &e1);
+    auto nblk = [](int rows) { return (rows + 255) / 256 * 8; }; // (32-row tiles padded to 8, one per XCD)
+    SkMats m, v;
+    m.W[0] = w[0].blocks, m.N[0] = w[0].rows, m.col[0] = 0, m.nb1 = nblk(w[0].rows);
+    m.W[1] = w[1].blocks, m.N[1] = w[1].rows, m.col[1] = w[0].rows;
+    v.W[0] = v.W[1] = w[2].blocks, v.N[0] = v.N[1] = w[2].rows, v.col[0] = v.col[1] = w[0].rows + w[1].rows, v.nb1 = nblk(w[2].rows);
+    const int bv = m.nb1 + nblk(w[1].rows);
+#define SK3_L(TA, TV) hipExtLaunchKernelGGL((k_gemm_kq32_3<TA, TV>), dim3(bv + v.nb1), dim3(SK_T), 0, s, e0, e1, 0, m, v, bv, w[0].bstride, \
+                                            w[2].bstride, w[0].cols, xq, xs, ldx, M, out, ldo, mode)
+    if (w[0].type == GW_Q6_K) SK3_L(GW_Q6_K, GW_Q6_K);
+    else if (w[2].type == GW_Q6_K) SK3_L(GW_Q4_K, GW_Q6_K);
+    else SK3_L(GW_Q4_K, GW_Q4_K);
+#undef SK3_L
+    return (int)hipGetLastError();
 }
 
 int gw_k_matmul(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int M, float *out, int ldo, int mode, hipStream_t s) {

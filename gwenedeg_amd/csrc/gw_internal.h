@@ -456,6 +456,7 @@ int gw_k_matmul(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int 
  * 9 .. 32 rows); else -1, nothing launched */
 int gw_k_matmul2(const GwMat *a, const GwMat *b, int col_b, const int8_t *xq, const float *xs, int ldx, int M, float *out,
                  int ldo, int mode, hipStream_t s);
+int gw_k_matmul3(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int M, float *out, int ldo, int mode, hipStream_t s);
 
 #ifdef __cplusplus
 }

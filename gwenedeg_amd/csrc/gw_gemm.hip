@@ -1130,7 +1130,8 @@ __global__ __launch_bounds__(SK_T * SB, SB == 1 ? 2 : 1) void k_gemm_kq32(SkMats
 }
 
 // two matrices of type TA (mats; blocks [0, bv)) and a third of type TV (mv; blocks from bv on) of one width: a layer's
-// q, k and v. v has few tiles (1,024 rows: 32 blocks) and as a launch of its own took as long as q and k beside it
+// q, k and v. v has few tiles (1,024 rows: 32 blocks) and as a launch of its own took as long as q and k: 4B widths, 32 rows,
+// us: Q4_K q + k 11.7 and Q6_K v 12.9, here 14.0
 template <int TA, int TV>
 __global__ __launch_bounds__(SK_T, 2) void k_gemm_kq32_3(SkMats mats, SkMats mv, int bv, int bstride, int bstride_v, int K,
                                                          const int8_t *__restrict__ X, const float *__restrict__ XS, int ldx,
@@ -1277,16 +1278,19 @@ __global__ __launch_bounds__(512, 4) void k_gemm_kql(SkMats mats, int bstride, i
 //   100 rows: Q6_K 2,560 x 9,728 145 -> 60; Q4_K 4,096 x 2,560 42 -> 16; 40 rows: 44 -> 18 (2,560 x 4,096), 38 -> 12 (1,024)
 //   32 rows: Q6_K 151,936 x 2,560 204 -> 133; Q4_K 19,456 x 2,560 25.7 -> 21.8; 8 rows: 194 -> 125, 28.1 -> 19.4
 template <int TYPE>
-__global__ __launch_bounds__(256, TYPE == GW_Q5_K ? 4 : 5) void k_gemm_kqt(SkMats mats, int bstride, int K, const int8_t *__restrict__ X,
-                                                     const float *__restrict__ XS, int ldx, int M, float *out, int ldo,
-                                                     int mode, int MT) {
+constexpr int KT_STG = 8192 + (KL_PPR(TYPE) * 32 + 63) / 64 * 1024 + 1024; // a stage: X codes, W super-blocks, X scales
+#define KT_XXR 80 // bytes per row of (xs, xf) pairs
+template <int TYPE>
+constexpr int KT_LDS = 2 * KT_STG<TYPE> + (TYPE == GW_Q6_K ? 0 : 32 * KT_XXR);
+template <int TYPE>
+__device__ __forceinline__ void kqt_block(uint8_t *sl, int bx, const SkMats &mats, int bstride, int K, const int8_t *__restrict__ X,
+                                          const float *__restrict__ XS, int ldx, int M, float *out, int ldo, int mode, int MT) {
     constexpr int PPR = KL_PPR(TYPE), PX = 8, PW = (PPR * 32 + 63) / 64, PT = PX + PW + 1, PPW = (PT + 3) / 4;
-    constexpr int OW = 8192, OXS = OW + PW * 1024, STG = OXS + 1024, XXR = 80; // (XXR: bytes per row of (xs, xf) pairs)
+    constexpr int OW = 8192, OXS = OW + PW * 1024, STG = KT_STG<TYPE>, XXR = KT_XXR;
     constexpr int PB = (TYPE == GW_Q4_K ? GW_Q4K_BYTES : TYPE == GW_Q5_K ? GW_Q5K_BYTES : GW_Q6K_DEV) / 16;
-    __shared__ __align__(16) uint8_t sl[2 * STG + (TYPE == GW_Q6_K ? 0 : 32 * XXR)];
     uint8_t *const xx = sl + 2 * STG;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l16 = lane & 15, q4 = lane >> 4;
-    const int mi = blockIdx.x >= mats.nb1, b = blockIdx.x - (mi ? mats.nb1 : 0), j = b >> 3, N = mats.N[mi];
+    const int mi = bx >= mats.nb1, b = bx - (mi ? mats.nb1 : 0), j = b >> 3, N = mats.N[mi];
     const int n0 = ((j / MT) * 8 + (b & 7)) * 32, m0 = (j % MT) * 32, S = K >> 8, gx = ldx >> 5;
     if (n0 >= N) return; // (the grid's padding to 8 column tiles per XCD)
     const int rowb = S * bstride;
@@ -1426,6 +1430,26 @@ __global__ __launch_bounds__(256, TYPE == GW_Q5_K ? 4 : 5) void k_gemm_kqt(SkMat
             *o = mode == 1 ? *o + acc[r] : acc[r];
         }
     }
+}
+
+template <int TYPE>
+__global__ __launch_bounds__(256, TYPE == GW_Q5_K ? 4 : 5) void k_gemm_kqt(SkMats mats, int bstride, int K, const int8_t *__restrict__ X,
+                                                     const float *__restrict__ XS, int ldx, int M, float *out, int ldo,
+                                                     int mode, int MT) {
+    __shared__ __align__(16) uint8_t sl[KT_LDS<TYPE>];
+    kqt_block<TYPE>(sl, (int)blockIdx.x, mats, bstride, K, X, XS, ldx, M, out, ldo, mode, MT);
+}
+
+// a layer's q, k (Q4_K, mats) and v (Q6_K, mv: blocks [0, bv), first, as theirs take longest): v alone was two blocks per CU
+// where five fit. 512 rows at the 4B widths, us: q + k 47.2 and v 19.5, here 59.7
+__global__ __launch_bounds__(256, 5) void k_gemm_kqt_3(SkMats mats, SkMats mv, int bv, int bstride, int bstride_v, int K,
+                                                       const int8_t *__restrict__ X, const float *__restrict__ XS, int ldx, int M,
+                                                       float *out, int ldo, int mode, int MT) {
+    __shared__ __align__(16) uint8_t sl[KT_LDS<GW_Q6_K> > KT_LDS<GW_Q4_K> ? KT_LDS<GW_Q6_K> : KT_LDS<GW_Q4_K>];
+    if ((int)blockIdx.x < bv)
+        kqt_block<GW_Q6_K>(sl, (int)blockIdx.x, mv, bstride_v, K, X, XS, ldx, M, out, ldo, mode, MT);
+    else
+        kqt_block<GW_Q4_K>(sl, (int)blockIdx.x - bv, mats, bstride, K, X, XS, ldx, M, out, ldo, mode, MT);
 }
 
 // --------------------------------------------------------------------------------------------- K-quants
@@ -2307,10 +2331,32 @@ int gw_k_matmul2(const GwMat *a, const GwMat *b, int col_b, const int8_t *xq, co
     return -1;
 }
 
+static int kqt3_takes(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int M) {
+    // q, k of Q4_K beside v of Q6_K above 32 rows, where k_gemm_kqt takes both launches (q and k as k_gemm_kql: they stay there)
+    return M > 32 && w[0].type == GW_Q4_K && w[1].type == GW_Q4_K && w[2].type == GW_Q6_K && w[1].cols == w[0].cols &&
+           w[2].cols == w[0].cols && w[0].bstride == w[1].bstride && !((uintptr_t)w[1].blocks & 15) &&
+           kql_takes(&w[0], w[0].rows + w[1].rows, xq, xs, ldx, M) == 1 && kql_takes(&w[2], w[2].rows, xq, xs, ldx, M) == 1;
+}
+
+static int launch_kqt3(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int M, float *out, int ldo, int mode, hipStream_t s) {
+    hipEvent_t e0, e1;
+    gw_take_launch_events(&e0, &e1);
+    const int mt = (M + 31) / 32;
+    auto nblk = [&](int rows) { return (rows + 255) / 256 * 8 * mt; }; // (column tiles padded to 8 per XCD)
+    SkMats m, v;
+    m.W[0] = w[0].blocks, m.N[0] = w[0].rows, m.col[0] = 0, m.nb1 = nblk(w[0].rows);
+    m.W[1] = w[1].blocks, m.N[1] = w[1].rows, m.col[1] = w[0].rows;
+    v.W[0] = v.W[1] = w[2].blocks, v.N[0] = v.N[1] = w[2].rows, v.col[0] = v.col[1] = w[0].rows + w[1].rows, v.nb1 = nblk(w[2].rows);
+    hipExtLaunchKernelGGL(k_gemm_kqt_3, dim3(v.nb1 + m.nb1 + nblk(w[1].rows)), dim3(256), 0, s, e0, e1, 0, m, v, v.nb1, w[0].bstride,
+                          w[2].bstride, w[0].cols, xq, xs, ldx, M, out, ldo, mode, mt);
+    return (int)hipGetLastError();
+}
+
 int gw_k_matmul3(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int M, float *out, int ldo, int mode, hipStream_t s) {
-    /* w[0], w[1] (of one type) and w[2], side by side in out's columns, in one launch where k_gemm_kq32 takes all three; else
-     * -1 and nothing launched. Every block is resident at once: w[0] and w[1] have at most a tile per CU (more go to
+    /* w[0], w[1] (of one type) and w[2], side by side in out's columns, in one launch where k_gemm_kqt takes all three
+     * (kqt3_takes), or k_gemm_kq32; else -1 and nothing launched. k_gemm_kq32: every block is resident at once: w[0] and w[1] have at most a tile per CU (more go to
      * k_gemm_kqt), w[2] too, and a CU holds two blocks */
+    if (kqt3_takes(w, xq, xs, ldx, M)) return launch_kqt3(w, xq, xs, ldx, M, out, ldo, mode, s);
     for (int i = 0; i < 3; i++)
         if (!kq32_takes(&w[i], M) || w[i].cols != w[0].cols) return -1;
     if (w[0].type != w[1].type || w[0].bstride != w[1].bstride || (w[0].type == GW_Q6_K && w[2].type != GW_Q6_K) || g_kq16 || g_kq32_nqr ||

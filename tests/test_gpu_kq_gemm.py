@@ -51,19 +51,19 @@ def test_lds_copied_kq_gemm_bitexact(dev, typ, N, K, M):
     assert (got[M] == 7.0).all()
 
 
-# q, k and v of a layer in one launch (9 .. 32 rows): each pair of types it takes, and one it leaves to launches of their own
-# (Q6_K q / k beside Q4_K v); k and v of one tile and of several
+# q, k and v of a layer in one launch (9 .. 32 rows: k_gemm_kq32_3, above: k_gemm_kqt_3): each pair of types they take, and
+# those they leave to launches of their own (Q6_K q / k beside Q4_K v); k and v of one tile and of several
 @pytest.mark.parametrize("typ,typ_v", [(12, 14), (12, 12), (14, 14), (14, 12)])
-@pytest.mark.parametrize("rows,heads,kv", [(9, 2, 1), (32, 6, 2), (17, 16, 8)])
+@pytest.mark.parametrize("rows,heads,kv", [(9, 2, 1), (32, 6, 2), (17, 16, 8), (33, 2, 1), (65, 16, 8)])
 def test_kq_qkv_launch_equals_oracle(dev, tmp_path, typ, typ_v, rows, heads, kv):
     _, gw = dev
     from oracle import oracle as orc
     from gwenedeg_amd import synth
     path = synth.write_gguf(str(tmp_path / "m.gguf"), "tiny_kq", seed=8, type_default=typ, type_v=typ_v, dim=768, n_heads=heads,
                             n_kv_heads=kv)
-    m, so = gw.Model(path, ctx_len=64), orc.Model(path, cap=64).seq()
+    m, so = gw.Model(path, ctx_len=80), orc.Model(path, cap=80).seq()
     ids = np.random.default_rng(rows).integers(0, m.vocab, rows).astype(np.int32)
     ref = np.stack([so.forward(int(t)) for t in ids])
-    got = m.ctx(max_batch=32).prefill(m.seq(64), ids, mode=gw.RQ_LOGITS_ALL)
+    got = m.ctx(max_batch=80).prefill(m.seq(80), ids, mode=gw.RQ_LOGITS_ALL)
     assert np.array_equal(np.ascontiguousarray(got, np.float32).view(np.uint32), ref.astype(np.float32).view(np.uint32)), \
         f"max diff {np.abs(got - ref).max()}"

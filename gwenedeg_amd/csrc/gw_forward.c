@@ -445,7 +445,6 @@ static int ctx_meta(RqCtx *c, size_t bytes) {
 static int ctx_lg(RqCtx *c, size_t rows) {
     if (rows <= c->lg_h_rows) return RQ_OK;
     if (c->lg_h) hipHostFree(c->lg_h);
-    if (c->g_h) hipHostFree(c->g_h);
     c->lg_h = NULL;
     c->lg_h_rows = 0;
     HIPCHK(c, "hipHostMalloc (logits)", hipHostMalloc((void **)&c->lg_h, rows * c->m->vocab * sizeof(float), hipHostMallocDefault));

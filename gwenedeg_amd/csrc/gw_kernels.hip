@@ -627,8 +627,9 @@ __global__ __launch_bounds__(AQ_T) void k_attn_q(const int4 *__restrict__ items,
 // that reach it: part[(row * nh + h) * pstride + kb * (hd + 2)] = o[hd] (unnormalized), m, l. Vector v = (row
 // r0 + v / kv_mul, head g * kv_mul + v % kv_mul) over positions 0..pos(row).
 // The fma chains run on the matrix cores: v_mfma_f32_16x16x4_f32 is four fmas in k order, each rounded once and with
-// denormals flushed as the VALU's in this build (a probe of a million chains over six ranges of values, denormals among
-// them, found every result equal), at twice the VALU's rate and without its operand broadcasts. What bounds an item is
+// denormals flushed as the VALU's in this build (tests/test_gpu_attention.py holds the kernels to it where flushing decides
+// the bits; a chain ending on -0 gets +0 from the zero products behind its row, which the combine and the quantizer do not
+// tell apart), at twice the VALU's rate and without its operand broadcasts. What bounds an item is
 // those MFMAs (2 x 128 per wave at 32 cycles: 3.4 us per CU and item at 2.4 GHz).
 //   scores: wave w takes positions 64 w ..; A = K (row i of MFMA u: position 64 w + 4 i + u, a lane's 8 bytes of a dim
 //     are the rows of 4 MFMAs; k: 4 consecutive dims), B = the vectors: 8 MFMAs per chunk of 32 dims, the chunks

@@ -723,6 +723,11 @@ void or_attention_block(float *o, float *ml, const float *q, const uint16_t *kc,
     attention_block(0, o, ml, q, kc, vc, n, b, h, n_kv, hd, scale);
 }
 
+void or_attention_block_bf16(float *o, float *ml, const float *q, const uint16_t *kc, const uint16_t *vc, int n, int b, int h,
+                             int n_kv, int hd, float scale) {
+    attention_block(1, o, ml, q, kc, vc, n, b, h, n_kv, hd, scale);
+}
+
 void or_att_combine(float *out, int nb, const float *part, size_t stride, int hd) {
     /* forward.c:1405-1431 */
     if (nb == 1) {

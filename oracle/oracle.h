@@ -36,6 +36,8 @@ void or_attention(float *out, const float *q, const uint16_t *kc, const uint16_t
 /* the partial result of block b (positions 256 b .. min(n, 256 b + 256) - 1): o[hd] unnormalized, ml = {m, l} */
 void or_attention_block(float *o, float *ml, const float *q, const uint16_t *kc, const uint16_t *vc, int n, int b, int h,
                         int n_kv, int hd, float scale);
+void or_attention_block_bf16(float *o, float *ml, const float *q, const uint16_t *kc, const uint16_t *vc, int n, int b, int h,
+                             int n_kv, int hd, float scale); /* (the bf16 caches' tiles) */
 void or_att_combine(float *out, int nb, const float *part, size_t stride, int hd); /* forward.c:1405-1431 */
 
 /* norms, RoPE, SwiGLU (forward.c:886-901, :1248-1284, :1953-1958) */

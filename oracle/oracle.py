@@ -47,6 +47,7 @@ def lib() -> ctypes.CDLL:
             "or_kv_tile": (ctypes.c_size_t, [I, I, I, I]),
             "or_attention": (None, [P, P, P, P, I, I, I, I, F]),
             "or_attention_block": (None, [P, P, P, P, P, I, I, I, I, I, F]),
+            "or_attention_block_bf16": (None, [P, P, P, P, P, I, I, I, I, I, F]),
             "or_att_combine": (None, [P, I, P, ctypes.c_size_t, I]),
             "or_rms_scale": (F, [P, I]),
             "or_rsqrt_ref": (F, [F]),

@@ -168,12 +168,13 @@ def test_device_argmax(gw, synth_models):
 
 
 @pytest.mark.parametrize("shape,n_prompt,steps", [("tiny", 9, 40), ("tiny_hd64", 250, 20), ("tiny_gqa4", 1000, 40),
-                                                  ("tiny_kq", 5, 6)])
+                                                  ("tiny_kq", 5, 6), ("tiny_kq", 250, 20), ("tiny_kq", 1000, 40),
+                                                  ("tiny_q5k", 250, 20), ("tiny_q3k", 5, 6)])
 def test_decode_greedy_equals_step_by_step(gw, synth_models, shape, n_prompt, steps):
     """gw_decode_greedy (tokens fed on the device, one wait) against gw_decode_argmax step by step and the host argmax
     of rq_decode's logits: the same tokens, the same cache (the logits of a later step agree bit for bit); across
     key-block boundaries (250 + 20 passes position 256, 1000 + 40 passes 1024: the combine past GW_GV_NBMAX blocks);
-    a K-quant model takes the step-by-step path"""
+    Q8_0 and Q4_K / Q5_K / Q6_K models run the fused sequence, a model with Q3_K the step-by-step path"""
     path = synth_models(shape)
     m = gw.Model(path, ctx_len=2048)
     c = m.ctx(max_batch=64, max_ctx=2048)
@@ -194,6 +195,25 @@ def test_decode_greedy_equals_step_by_step(gw, synth_models, shape, n_prompt, st
     a = c.decode(s1, 7)
     b = c.decode(s2, 7)
     assert _bits_equal(a, b)
+
+
+@pytest.mark.parametrize("shape", ["tiny_gqa4", "tiny_kq"])
+def test_decode_greedy_into_long_rows(gw, synth_models, shape):
+    """gw_decode_greedy across position 8,192, where 8 heads' blocks pass one per CU and the attention goes from
+    k_attn_decode to k_attn_decode4: the tokens and cache of gw_decode_argmax step by step and of one-row prompt passes"""
+    m = gw.Model(synth_models(shape), ctx_len=9216)
+    c = m.ctx(max_batch=2)
+    s1, s2, s3 = m.seq(9216), m.seq(9216), m.seq(9216)
+    for s in (s1, s2, s3):
+        s.fill_synthetic(8186, 5)
+    got = [int(t) for t in c.decode_greedy(s1, 3, 12)]
+    fed = [3] + got[:-1]
+    assert [c.decode_argmax(s2, t) for t in fed] == got
+    for i in range(0, 12, 2):  # (two rows per pass: the batched kernels)
+        lg = c.prefill(s3, np.array(fed[i:i + 2], np.int32), mode=gw.RQ_LOGITS_ALL)
+        assert [int(t) for t in np.argmax(lg, 1)] == got[i:i + 2]
+    a, b, d = (c.decode(s, 7) for s in (s1, s2, s3))
+    assert _bits_equal(a, b) and _bits_equal(a, d)
 
 
 @pytest.mark.parametrize("kvt", [3, 9, 0, 1, 5, 7])

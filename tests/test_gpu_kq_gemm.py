@@ -16,14 +16,15 @@ def dev():
 
 # 12 Q4_K, 13 Q5_K, 14 Q6_K. k_gemm_kqt: above 32 rows, one to several stages (K / 256), row and column remainders of its
 # 32 x 32 tiles; 6 .. 32 rows once its tiles are more than one per CU (8,193 weight rows); Q5_K from 9 rows. k_gemm_kql (Q4_K):
-# 64 x 128 blocks that fill the CUs (25,700 weight rows, 33 rows; 1 row past a block). 131,100-row
-# Q6_K at 33 rows keeps k_gemm_kq (4 blocks per CU)
+# 64 x 128 blocks that fill the CUs (25,700 weight rows, 33 rows; 1 row past a block: 25,601 at 65 and, with three stages, 9,601
+# at 129; 12,801 at 129 leave two fifths of a round empty: k_gemm_kqt). 131,100-row Q6_K at 33 rows keeps k_gemm_kq (4 blocks
+# per CU)
 @pytest.mark.parametrize("typ,N,K,M", [
     (12, 31, 256, 33), (12, 33, 512, 64), (12, 200, 2560, 65), (12, 1000, 768, 97),
     (13, 33, 256, 33), (13, 200, 1024, 9), (13, 70, 512, 32), (13, 129, 768, 70),
     (14, 1, 256, 33), (14, 33, 512, 40), (14, 200, 2560, 65), (14, 130, 9728, 36),
     (12, 8193, 256, 6), (12, 8193, 512, 32), (13, 8193, 256, 7), (14, 8193, 256, 6), (14, 8200, 512, 31),
-    (12, 25700, 256, 33), (12, 25601, 512, 65), (12, 12801, 768, 129),
+    (12, 25700, 256, 33), (12, 25601, 512, 65), (12, 12801, 768, 129), (12, 9601, 768, 129),
     (14, 131100, 256, 33)])
 def test_lds_copied_kq_gemm_bitexact(dev, typ, N, K, M):
     torch, gw = dev
@@ -65,5 +66,21 @@ def test_kq_qkv_launch_equals_oracle(dev, tmp_path, typ, typ_v, rows, heads, kv)
     ids = np.random.default_rng(rows).integers(0, m.vocab, rows).astype(np.int32)
     ref = np.stack([so.forward(int(t)) for t in ids])
     got = m.ctx(max_batch=80).prefill(m.seq(80), ids, mode=gw.RQ_LOGITS_ALL)
+    assert np.array_equal(np.ascontiguousarray(got, np.float32).view(np.uint32), ref.astype(np.float32).view(np.uint32)), \
+        f"max diff {np.abs(got - ref).max()}"
+
+
+# w1 and w3 in one launch of k_gemm_kql (33 rows: 100 blocks of 128 weight rows each, 200 of the 256 CUs) and of k_gemm_kqt (80
+# each), w2 of 50 and of 40 super-blocks
+@pytest.mark.parametrize("hidden", [12800, 10240])
+def test_kq_ffn_launch_equals_oracle(dev, tmp_path, hidden):
+    _, gw = dev
+    from oracle import oracle as orc
+    from gwenedeg_amd import synth
+    path = synth.write_gguf(str(tmp_path / "m.gguf"), "tiny_kq", seed=9, dim=256, hidden=hidden, n_heads=2, n_kv_heads=1, n_layers=1)
+    m, so = gw.Model(path, ctx_len=64), orc.Model(path, cap=64).seq()
+    ids = np.random.default_rng(hidden).integers(0, m.vocab, 33).astype(np.int32)
+    ref = np.stack([so.forward(int(t)) for t in ids])
+    got = m.ctx(max_batch=64).prefill(m.seq(64), ids, mode=gw.RQ_LOGITS_ALL)
     assert np.array_equal(np.ascontiguousarray(got, np.float32).view(np.uint32), ref.astype(np.float32).view(np.uint32)), \
         f"max diff {np.abs(got - ref).max()}"

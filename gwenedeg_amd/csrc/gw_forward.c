@@ -6,11 +6,11 @@
  *   attention partials per (row block, kv head, 256-position block) -> combine + quantize -> wo matmul ->
  *   residual + rmsnorm + quantize -> w1 / w3 matmul -> SwiGLU + quantize -> w2 matmul
  *   -> final residual + rmsnorm + quantize of the selected rows -> classifier -> logits to the host.
- * A one-row pass of an all-Q8_0 model (decode) runs the fused sequence instead: per layer qkv matmul (rmsnorm +
- * quantize in its prologue) -> QK-norm + RoPE + K / V store -> attention partials -> wo matmul (combine + quantize in
- * its prologue, + residual) -> w1 / w3 matmul (rmsnorm + quantize in its prologue, SwiGLU in its epilogue) -> w2 matmul
- * (quantize in its prologue, + residual), and the classifier's GEMV computes the final rmsnorm + quantize itself: the
- * same arithmetic, four kernels fewer per layer.
+ * A one-row pass of an all-Q8_0 model, or of a Q4_K / Q5_K / Q6_K one (decode), runs the fused sequence instead: per
+ * layer qkv matmul (rmsnorm + quantize in its prologue) -> attention partials (QK-norm, RoPE and K / V store inside) -> wo
+ * matmul (combine + quantize in its prologue, + residual) -> w1 / w3 matmul (rmsnorm + quantize in its prologue, SwiGLU in
+ * its epilogue) -> w2 matmul (quantize in its prologue, + residual), and the classifier's GEMV computes the final rmsnorm +
+ * quantize itself: the same arithmetic, five launches per layer.
  * The same kernels run every row whatever its batch-mates (decode is a one-row pass), and each output is computed
  * whole in a fixed order, so a sequence's results do not depend on what it is batched with (runq.h:22-24).
  * Errors: every argument is validated before any device work (forward.c:3775-3800), so a failed pass changes nothing;
@@ -1244,8 +1244,8 @@ int rq_prefill(RqCtx *c, RqSeq *s, const int *tokens, int n, int mode, float *ou
 
 int gw_ctx_gemv_sweep(RqCtx *c, int reps, double *seconds, double *bytes, int *launches) {
     /* the weight matmuls of one decode step (every layer's q / k / v, wo, w1 / w3, w2, then the classifier), launched
-     * as a one-row pass launches them (an all-Q8_0 model: the fused GEMVs with their prologues and epilogues, the
-     * attention combine over one key block), back to back on the context's stream, reps times, between two HIP
+     * as a one-row pass launches them (an all-Q8_0 model, or a Q4_K / Q5_K / Q6_K one: the fused GEMVs with their prologues
+     * and epilogues, the attention combine over one key block), back to back on the context's stream, reps times, between two HIP
      * events: the device time of the decode path's weight streaming without the other kernels between them. The
      * inputs are whatever the context's buffers hold (the kernels' time does not depend on the values); the outputs go
      * to the context's scratch rows. *bytes: the file-format bytes of those weights per sweep (Q8_0 34 / 32, Q4_K

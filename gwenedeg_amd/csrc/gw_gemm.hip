@@ -1151,9 +1151,9 @@ __global__ __launch_bounds__(SK_T, 2) void k_gemm_kq32_3(SkMats mats, SkMats mv,
 // q x (int8 MFMA), and one outer-product MFMA (v_mfma_f32_32x32x1_f32, two blocks; each result one fp32 product rounded
 // once, as the VALU's multiply) gives xs f0 (f0 = d sc_j) and xf f1 (f1 = dmin m_j, xf = xs (float) sum x, the pairs (xs,
 // xf) made once per stage by the block's threads): term = (xs f0) (float) I - xf f1 (kquants.h:86-109), val = val + term
-// in group order. The VALU bounds it (the fp32 MFMA issues through its pipe too): 4 instructions per output and group and
-// one in two for the products, 370 of them per 32 x 32 tile and group with the unpacking; at 4 waves per SIMD they issue
-// 83 % of the cycles. k_gemm_kq (unpacks into LDS between two barriers per half super-block, 8 instructions per output and
+// in group order. The VALU bounds it (the fp32 MFMA issues through its pipe too): per wave, 32 x 32 tile and group 75
+// instructions of 4 cycles (64 of them the fold's 4 per output, the rest the unpacking) and the products' MFMA of 64, about 365
+// issue cycles; at 4 waves per SIMD they fill 83 % of the time. k_gemm_kq (unpacks into LDS between two barriers per half super-block, 8 instructions per output and
 // group) -> here, us per launch at 512 rows: 19,456 x 2,560 165 -> 142, 9,728 x 2,560 110 -> 86, 4,096 x 2,560 53 -> 37
 // LDS: chunk c of X row r at c ^ (r % 16) of the row's 16; W rows 144 bytes apart (the 16 rows of a read on distinct banks)
 #define KL_PPR(T) ((T) == GW_Q4_K ? 9 : (T) == GW_Q5_K ? 11 : 14) // 16-byte pieces of a super-block
@@ -2212,8 +2212,9 @@ static int q8l_width(int N, int M, int K) {
 }
 
 static bool kq32_takes(const GwMat *w, int M) {
-    // K-quants, 9 .. 32 rows: the 32-row GEMM with the groups spread over a block's waves (a matrix of 32768 rows or
-    // more, the classifier: the 128-column MFMA GEMM, a block for every compute unit)
+    // K-quants, 9 .. 32 rows: the 32-row GEMM with the groups spread over a block's waves, where kql_takes, which is asked
+    // first, leaves them: at most a 32-row tile per CU, or inputs that its 16-byte copies do not take (then a matrix of 32768
+    // rows or more, the classifier, goes to the 128-column MFMA GEMM, a block for every compute unit)
     return (w->type == GW_Q4_K || w->type == GW_Q6_K) && M > 8 && M <= 32 && !g_tile_rows && w->rows < 32768;
 }
 
@@ -2279,8 +2280,12 @@ static int kql_takes(const GwMat *w, int rows, const int8_t *xq, const float *xs
     // one per CU, from 6 rows (us, GEMV / k_gemm_kqt: Q4_K 19,456 x 2,560 at 5 rows 19.0 / 19.4, 6 19.6 / 18.4, 8 28 / 19;
     // k_gemm_kq32 / k_gemm_kqt at 32 rows: 9,728 x 2,560 (304 tiles) 17.2 / 15.6, 5,120 x 2,560 (160) 11.1 / 13.0), and for
     // Q5_K, which k_gemm_kq32 does not take, above 8. Above 32 rows: k_gemm_kql (Q4_K) where its 64 x 128 blocks fill at
-    // least 78 % of the CU rounds they take (k_gemm_kql / k_gemm_kqt: 256 blocks 37 / 42, 304 54.9 / 50.9, 320 53.8 / 51.2, 608
-    // 86 / 93, 1,216 142 / 178), else k_gemm_kqt; Q6_K where k_gemm_kq's 64 x 128 tiles are 4 per CU or more stays there
+    // least 78 % of the CU rounds they take, else k_gemm_kqt. The two cross at another fill in each round: in the first near
+    // 90 %, in the second at 72 %, in the third at 75 % (K 2,560, 512 rows, us, k_gemm_kql / k_gemm_kqt: 176 blocks (69 %)
+    // 32.3 / 29.9, 200 (78 %) 32.6 / 32.5, 224 (88 %) 33.6 / 32.9, 240 34.5 / 36.4; 336 (66 %) 51.5 / 48.2, 368 (72 %)
+    // 51.0 / 51.8, 400 (78 %) 51.6 / 55.9; 560 (73 %) 77.4 / 76.7, 592 (77 %) 77.5 / 79.9, 608 78.2 / 81.0, 640 78.0 / 84.9;
+    // 64 rows, 192 blocks 35.4 / 30.2, 200 35.4 / 33.0), so one line costs up to 7 % on either side of it; 1,216 blocks
+    // 142 / 178. Q6_K where k_gemm_kq's 64 x 128 tiles are 4 per CU or more stays there
     // (16,384 x 2,560 at 512 rows 171 / 208; at 256, below that, 100 / 102)
     if ((w->type != GW_Q4_K && w->type != GW_Q5_K && w->type != GW_Q6_K) || g_tile_rows ||
         (((uintptr_t)w->blocks | (uintptr_t)xq | (uintptr_t)xs) & 15) || ldx % 128 || (size_t)128 * (w->cols >> 8) * w->bstride >= ((size_t)1 << 30))
@@ -2354,8 +2359,8 @@ static int launch_kqt3(const GwMat *w, const int8_t *xq, const float *xs, int ld
 
 int gw_k_matmul3(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int M, float *out, int ldo, int mode, hipStream_t s) {
     /* w[0], w[1] (of one type) and w[2], side by side in out's columns, in one launch where k_gemm_kqt takes all three
-     * (kqt3_takes), or k_gemm_kq32; else -1 and nothing launched. k_gemm_kq32: every block is resident at once: w[0] and w[1] have at most a tile per CU (more go to
-     * k_gemm_kqt), w[2] too, and a CU holds two blocks */
+     * (kqt3_takes), or k_gemm_kq32; else -1 and nothing launched. k_gemm_kq32: every block is resident at once: w[0] and
+     * w[1] have at most a tile per CU (more go to k_gemm_kqt), w[2] too, and a CU holds two blocks */
     if (kqt3_takes(w, xq, xs, ldx, M)) return launch_kqt3(w, xq, xs, ldx, M, out, ldo, mode, s);
     for (int i = 0; i < 3; i++)
         if (!kq32_takes(&w[i], M) || w[i].cols != w[0].cols) return -1;
@@ -2420,9 +2425,10 @@ int gw_k_matmul(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int 
     const int kern = kql_takes(w, w->rows, xq, xs, ldx, M);
     if (kern) return launch_kql(kern, w, NULL, 0, xq, xs, ldx, M, out, ldo, mode, s);
     if (kq32_takes(w, M)) return launch_kq32(w, NULL, 0, xq, xs, ldx, M, out, ldo, mode, s);
-    // K-quants above 32 rows: the MFMA GEMM where it has 64 blocks or more (a block streams its 128 rows' full K in
-    // order, so a narrow matrix leaves the device idle) or its row tile is forced, else the batched GEMV in passes of
-    // 8 rows
+    // what kql_takes and kq32_takes leave of the K-quants above 8 rows: k_gemm_kq where it has 64 blocks or more (a block
+    // streams its 128 rows' full K in order, so a narrow matrix leaves the device idle) or its row tile is forced, else the
+    // batched GEMV in passes of 8 rows. The other types come here always, Q6_K where k_gemm_kq has four tiles per CU; Q4_K and
+    // Q5_K only with inputs that are not 16-byte aligned or a forced row tile
     if (GW_IS_KQ(w->type) && M > 8 && (g_tile_rows || (size_t)((w->rows + GN - 1) / GN) * ((M + 31) / 32) >= 64)) {
         hipEvent_t e0, e1;
         gw_take_launch_events(&e0, &e1);

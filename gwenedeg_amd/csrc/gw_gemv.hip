@@ -22,6 +22,8 @@
 #include "gw_device.h"
 
 enum { GV_Q = 0, GV_NORM = 1, GV_QF = 2, GV_COMBINE = 3 };
+static_assert((int)GW_GK_Q == GV_Q && (int)GW_GK_NORM == GV_NORM && (int)GW_GK_QF == GV_QF && (int)GW_GK_COMBINE == GV_COMBINE,
+              "gw_k_gemvk's prologues");
 #define GV_NBMAX GW_GV_NBMAX
 
 struct GvArgs {
@@ -394,7 +396,6 @@ struct GkArgs {
     const int8_t *xq;
     const float *xs, *x, *nw, *part;
     int pstride, hd, nb;
-    float inv_k;
     float *out;
 };
 
@@ -839,7 +840,7 @@ static int gk_plan(int pro, const GwMat *w, int nmat, int swiglu, GkArgs *a, int
         if (swiglu || a->run < 1) return (int)hipErrorInvalidValue;
     }
     const size_t terms = (size_t)(rows <= most ? rows : a->run) * PS * 4, row = pro == GV_NORM ? (size_t)16 * (4 * rms_nf(K / 64) + 4) * 4 : 0;
-    a->nseg = ns, a->K = K, a->swiglu = swiglu, a->inv_k = 1.0f / (float)K;
+    a->nseg = ns, a->K = K, a->swiglu = swiglu;
     *nblocks = b0;
     *lds = (size_t)K + K / 16 * 4 + 2 * G * 4 + (terms > row ? terms : row);
     return 0;

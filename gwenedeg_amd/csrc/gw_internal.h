@@ -439,7 +439,7 @@ typedef struct {
     const float *xs, *x, *nw, *part;
     int pstride, hd, nb;
 } GwGkIn;
-enum { GW_GK_Q = 0, GW_GK_NORM = 1, GW_GK_QF = 2, GW_GK_COMBINE = 3 }; /* (gw_gemv.hip's prologues) */
+enum { GW_GK_Q = 0, GW_GK_NORM = 1, GW_GK_QF = 2, GW_GK_COMBINE = 3 }; /* (gw_gemv.hip's prologues, which it checks) */
 int gw_k_gemvk_ok(int pro, const GwMat *w, int nmat, int swiglu);
 int gw_k_gemvk(int pro, const GwMat *w, int nmat, int swiglu, const GwGkIn *in, float *out, int mode, hipStream_t s);
 
@@ -452,10 +452,13 @@ void gw_take_launch_events(hipEvent_t *a, hipEvent_t *b);
 /* the matmul dispatch (gw_gemm.hip): out[m * ldo + row] (+)= W row . X row m for M rows, any supported type */
 int gw_k_matmul(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int M, float *out, int ldo, int mode,
                 hipStream_t s);
-/* a and b (out from column col_b) in one launch where the kernel allows (two K-quant matrices of one type and width,
- * 9 .. 32 rows); else -1, nothing launched */
+/* a and b (out from column col_b) in one launch where one of the K-quant GEMMs takes both (one type and width: Q4_K and Q6_K
+ * from 9 rows, Q5_K too where k_gemm_kqt takes it; kql_takes, kq32_takes); else -1, nothing launched */
 int gw_k_matmul2(const GwMat *a, const GwMat *b, int col_b, const int8_t *xq, const float *xs, int ldx, int M, float *out,
                  int ldo, int mode, hipStream_t s);
+/* w[0], w[1] and w[2] (q, k and v: side by side in out's columns) in one launch: of one width, w[0] and w[1] of one type; 9 ..
+ * 32 rows Q4_K beside Q4_K or Q6_K, or Q6_K alone, above 32 rows Q4_K beside Q6_K, each where the kernels of their pair and of
+ * w[2] are the same (k_gemm_kq32, k_gemm_kqt); else -1, nothing launched */
 int gw_k_matmul3(const GwMat *w, const int8_t *xq, const float *xs, int ldx, int M, float *out, int ldo, int mode, hipStream_t s);
 
 #ifdef __cplusplus

@@ -287,8 +287,8 @@ int gw_forward_batch_device(RqCtx *c, const RqSegment *seg, int nseg);
 int gw_ctx_profile_enable(RqCtx *c, int on);
 
 /* The weight matmuls of one decode step (per layer q / k / v, wo, w1 / w3, w2; then the classifier), launched as a
- * one-row pass launches them (all-Q8_0 models: the fused GEMVs), back to back, reps times, timed with HIP events on
- * the context's stream: *seconds per sweep, *bytes = their file-format weight bytes (the algorithmic bytes of a decode
+ * one-row pass launches them (all-Q8_0 and Q4_K / Q5_K / Q6_K models: the fused GEMVs), back to back, reps times, timed with
+ * HIP events on the context's stream: *seconds per sweep, *bytes = their file-format weight bytes (the algorithmic bytes of a decode
  * step's weight streaming), *launches per sweep. Inputs are the context's buffers as they are (call it after a pass);
  * outputs go to its scratch rows. The counterpart of the reference's pass timing (rq_pass_times, runq.h:196-199) for
  * the GEMV alone */

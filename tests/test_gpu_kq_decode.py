@@ -48,3 +48,16 @@ def test_kq_decode_equals_oracle_and_prompt_rows(gw, tmp_path, over):
         rows = c.prefill(s, ids[:2], mode=gw.RQ_LOGITS_ALL)
         assert _bits_equal(one[0], rows[0]) and _bits_equal(one[1], rows[1]), f"{over}: position {n}"
         s.fill_synthetic(1279, 3)
+
+
+# the hidden row of a fused one-row pass (its final rmsnorm as a launch of its own, then the classifier on its codes) beside those
+# of a prompt pass
+@pytest.mark.parametrize("shape", ["tiny_kq", "tiny_q5k"])
+def test_kq_hidden_rows_equal_prompt_rows(gw, synth_models, shape):
+    m = gw.Model(synth_models(shape), ctx_len=64)
+    c, a, b = m.ctx(max_batch=8), m.seq(64), m.seq(64)
+    ids = np.random.default_rng(7).integers(0, m.vocab, 5).astype(np.int32)
+    rows, hid = c.prefill_hidden(a, ids, mode=gw.RQ_LOGITS_ALL)
+    for i, t in enumerate(ids):
+        lg, h = c.decode_hidden(b, int(t))
+        assert _bits_equal(lg, rows[i]) and _bits_equal(h, hid[i]), i
